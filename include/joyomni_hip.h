@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define JOY_ABI_VERSION 10
+#define JOY_ABI_VERSION 11
 
 #if defined(__GNUC__) || defined(__clang__)
 #define JOY_API __attribute__((visibility("default")))
@@ -330,6 +330,21 @@ JOY_API joy_status joy_fused_cached_kv_pack(const joy_bf16_view *key0, const joy
 JOY_API joy_status joy_attention_fwd(const joy_bf16_view *q, const joy_bf16_view *k, const joy_bf16_view *v,
                                      void *out, int64_t out_stride_token, int64_t num_heads, int64_t head_dim,
                                      float scale, void *stream);
+
+/*
+ * joy_attention_fwd with a caller-owned workspace: calls whose query blocks leave the last
+ * round of compute units partly idle then split the keys of that round over the idle ones and
+ * add the fp32 parts in key order in a second launch (results do not depend on timing; they
+ * differ from the unsplit call by the order of the softmax sums). joy_attention_workspace_size
+ * gives the bytes on the current device, 0 where the split does not pay. A null or smaller
+ * workspace runs the unsplit call. workspace: 16-byte aligned device memory, contents undefined
+ * before and after, in use until the call's kernels end.
+ */
+JOY_API int64_t joy_attention_workspace_size(int64_t q_len, int64_t k_len, int64_t num_heads);
+JOY_API joy_status joy_attention_fwd_workspace(const joy_bf16_view *q, const joy_bf16_view *k,
+                                     const joy_bf16_view *v, void *out, int64_t out_stride_token,
+                                     int64_t num_heads, int64_t head_dim, float scale, void *workspace,
+                                     int64_t workspace_bytes, void *stream);
 
 /*
  * (Layer|RMS)Norm + adaLN scale/shift.

@@ -114,17 +114,52 @@ __device__ __forceinline__ float xor32_sum(float v) {
 // straddle a head boundary moves the K / V tiles of both heads (LDS holds two heads' tiles);
 // qb_per_head >= 8 keeps it to two heads. Blocks past the list (last workgroup) compute on the
 // last valid block and store nothing.
+//
+// Key split (AttnSplit, split_plan): the groups past the last whole round of the chip can be cut
+// along the keys, a part per workgroup. A part leaves its unnormalised fp32 O and its running max
+// and sum in the workspace, and attn_combine adds a group's parts in key order. A workgroup takes
+// one part only: a loop over several in one workgroup costs 114 VGPR spills. What the kernel is
+// bound by stays as above (LDS operand reads and power); the split fills idle CUs. Measured against
+// the unsplit call: 512 x 8000 x 32 heads 179 -> 80 us, 859 x 5000 x 32 131 -> 98 us, 5000 x 5000 x 40
+// 571 -> 496 us, 3467 x 11267 x 32 636 -> 629 us. (wave is moved to a scalar register, so that the DMA's
+// LDS addresses are scalars: 250 -> 248 VGPRs with the split's code, 0.5-3 % faster unsplit.)
 constexpr int kWaves = 8;
-__global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int qb_per_head) {
+constexpr int kPartBlock = 64 * 64 + 64;        // floats per query block of a part: O, then m and l of 32 queries
+constexpr int kPartSlot = kWaves * kPartBlock;  // floats per part (one group)
+constexpr int kSplitMinTiles = 4;               // key tiles of a part: below, its prologue and epilogue dominate
+struct AttnSplit {
+  float* ws;         // [split_groups][parts] slots
+  int full_groups;   // the workgroups before the split ones: a whole group each
+  int split_groups;
+  int parts;         // parts per split group
+  int part_tiles;    // key tiles of each part but the last, which has what is left
+};
+
+__global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int qb_per_head, AttnSplit sp) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[2][2][2][kTileB];  // [buffer][head slot][K, V]
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ql = lane & 31, hf = lane >> 5;
   const int64_t Lq = a.q_len, Lk = a.k_len;
   const int nblocks = a.heads * qb_per_head;
-  const int blk0 = (int)blockIdx.x * kWaves;
-  const int head_lo = blk0 / qb_per_head;
-  const int head_hi = (min(blk0 + kWaves, nblocks) - 1) / qb_per_head;  // blk0 < nblocks
+  // this workgroup's group of query blocks and its key tiles [t0, t1)
+  const int64_t ntiles = (Lk + kBK - 1) / kBK;
+  int group = (int)blockIdx.x;
+  int slot = -1;
+  int64_t t0 = 0, t1 = ntiles;
+  if (group >= sp.full_groups) {
+    const int w = group - sp.full_groups;
+    // part 0 of every group first, then part 1, ... (the shorter last ones at the end); the quotient
+    // is uniform but computed on the VALU, so it is moved to a scalar register
+    const int part = __builtin_amdgcn_readfirstlane(w / sp.split_groups), g = w - part * sp.split_groups;
+    group = sp.full_groups + g;
+    slot = g * sp.parts + part;
+    t0 = (int64_t)part * sp.part_tiles;
+    t1 = min(ntiles, t0 + sp.part_tiles);
+  }
+  const int blk0 = group * kWaves;
+  const int head_lo = __builtin_amdgcn_readfirstlane(blk0 / qb_per_head);
+  const int head_hi = __builtin_amdgcn_readfirstlane((min(blk0 + kWaves, nblocks) - 1) / qb_per_head);  // blk0 < nblocks
   const bool straddle = head_hi != head_lo;
   const int blk = min(blk0 + wave, nblocks - 1);
   const bool active = blk0 + wave < nblocks;
@@ -210,7 +245,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int 
     for (int r = 3; r < 15; r += 2) m = fmaxf(fmaxf(m, s[r]), s[r + 1]);
     const float mt = xor32_max(fmaxf(m, s[15]));
     const float m_cand = mt * sl2;
-    st.m_new = fmaxf(m_run, m_cand);
+    // finite also where every score so far is -inf, so that such a tile adds nothing instead of NaN
+    st.m_new = fmaxf(fmaxf(m_run, m_cand), -3.0e38f);
     st.alpha = __builtin_amdgcn_exp2f(m_run - st.m_new);
     st.rs = 0.f;
 #pragma unroll
@@ -249,15 +285,14 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int 
     return __builtin_bit_cast(v4i, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
-  const int64_t ntiles = (Lk + kBK - 1) / kBK;
-  dma_tile(0, 0);
+  dma_tile(0, t0 * kBK);
   auto tile = [&](auto bufc, auto partc, int64_t t) {
     constexpr int buf = decltype(bufc)::value;
     constexpr bool partial = decltype(partc)::value;
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if (t + 1 < ntiles) dma_tile(buf ^ 1, (t + 1) * kBK);
+    if (t + 1 < t1) dma_tile(buf ^ 1, (t + 1) * kBK);
     const uint8_t* kt = lds[buf][hslot][0];
     const uint8_t* vt = lds[buf][hslot][1];
     const int64_t k0 = t * kBK;
@@ -323,8 +358,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int 
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  const int64_t nfull = Lk / kBK;
-  int64_t t = 0;
+  const int64_t nfull = min(t1, Lk / kBK);
+  int64_t t = t0;
   for (; t + 2 <= nfull; t += 2) {
     tile(IC<0>{}, std::false_type{}, t);
     tile(IC<1>{}, std::false_type{}, t + 1);
@@ -332,13 +367,22 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int 
   if (t < nfull) {
     tile(IC<0>{}, std::false_type{}, t);
     ++t;
-    if (t < ntiles) tile(IC<1>{}, std::true_type{}, t);
-  } else if (t < ntiles) {
+    if (t < t1) tile(IC<1>{}, std::true_type{}, t);
+  } else if (t < t1) {
     tile(IC<0>{}, std::true_type{}, t);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);
 
-  if (active && qrow < Lq) {
+  if (slot >= 0) {
+    float* pp = sp.ws + (int64_t)slot * kPartSlot + wave * kPartBlock;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4)
+        *(float4*)(pp + (db * 4 + r4) * 256 + lane * 4) =
+            make_float4(o[db][4 * r4], o[db][4 * r4 + 1], o[db][4 * r4 + 2], o[db][4 * r4 + 3]);
+    pp[64 * 64 + lane] = hf == 0 ? m_run : l_run;  // both halves hold their query's m and l
+  } else if (active && qrow < Lq) {
     const float inv = 1.0f / l_run;
     uint16_t* op = a.out + (int64_t)qrow * a.out_stride_token + (int64_t)head * kD;
 #pragma unroll
@@ -354,6 +398,82 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int 
   }
 }
 
+// Adds the parts of the split groups in key order: one 256-thread workgroup per query block, wave w
+// the 32 output columns of accumulator w of attn_fwd_d128, in the same lane layout.
+__global__ __launch_bounds__(256) void attn_combine(AttnArgs a, int qb_per_head, AttnSplit sp) {
+  const int lane = threadIdx.x & 63, db = threadIdx.x >> 6;
+  const int ql = lane & 31, hf = lane >> 5;
+  const int g = (int)blockIdx.x / kWaves, wave = (int)blockIdx.x % kWaves;
+  const int blk = (sp.full_groups + g) * kWaves + wave;
+  if (blk >= a.heads * qb_per_head) return;  // padding of the last group
+  const int head = blk / qb_per_head;
+  const int qrow = (blk - head * qb_per_head) * 32 + ql;
+  const float* pp = sp.ws + (int64_t)g * sp.parts * kPartSlot + wave * kPartBlock;
+  float4 o[4];
+#pragma unroll
+  for (int r4 = 0; r4 < 4; ++r4) o[r4] = *(const float4*)(pp + (db * 4 + r4) * 256 + lane * 4);
+  float m = pp[64 * 64 + ql], l = pp[64 * 64 + 32 + ql];
+  for (int p = 1; p < sp.parts; ++p) {
+    pp += kPartSlot;
+    const float mp = pp[64 * 64 + ql], lp = pp[64 * 64 + 32 + ql];
+    const float m_new = fmaxf(m, mp);
+    const float sa = __builtin_amdgcn_exp2f(m - m_new), sb = __builtin_amdgcn_exp2f(mp - m_new);
+    m = m_new;
+    l = l * sa + lp * sb;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const float4 x = *(const float4*)(pp + (db * 4 + r4) * 256 + lane * 4);
+      o[r4].x = o[r4].x * sa + x.x * sb;
+      o[r4].y = o[r4].y * sa + x.y * sb;
+      o[r4].z = o[r4].z * sa + x.z * sb;
+      o[r4].w = o[r4].w * sa + x.w * sb;
+    }
+  }
+  if (qrow >= a.q_len) return;
+  const float inv = 1.0f / l;
+  uint16_t* op = a.out + (int64_t)qrow * a.out_stride_token + (int64_t)head * kD;
+#pragma unroll
+  for (int r4 = 0; r4 < 4; ++r4) {
+    uint2 w;
+    w.x = pack_bf16x2(o[r4].x * inv, o[r4].y * inv);
+    w.y = pack_bf16x2(o[r4].z * inv, o[r4].w * inv);
+    *(uint2*)(op + db * 32 + 8 * r4 + 4 * hf) = w;
+  }
+}
+
+// Key split of the last, partial round: the `rest` groups past the last whole round of the chip
+// would take a whole round's time on a part of it. Each is cut into `s` equal parts, s * rest of
+// them in one workgroup each at the same time, and one shorter rest; the CUs that the s * rest
+// parts leave idle take the rests, at most k = ceil(rest / idle) of them each. With parts of
+// k / (1 + k s) of the keys a CU's k rests take as long as one part, so the round ends after that
+// share of its time (rest = 180 of 256 CUs: s = 1, k = 3, 3/4; the least any split reaches is
+// 180 / 256).
+// The split costs the parts' way to memory and back (133 KB each) and a second launch, and the more
+// CUs the unsplit round keeps busy, the less it has to give: power sets the clock, so a round on
+// part of the chip runs faster per tile. It is taken when it takes at least 5 + 26 rest / cus key
+// tiles off the round. Measured (unsplit, split; tiles taken off, rest): 512 x 600 x 32 22.2, 22.1 us
+// (8, 64); x 1000 30.4, 24.4 (12, 64); 859 x 859 30.7, 35.8 (8, 108); x 2000 58.6, 50.9 (18, 108);
+// 1371 x 2731 78.3, 83.1 (11, 172); x 5000 132, 127 (20, 172); 7367 x 3900 430, 434 (20, 156); x 7367
+// 850, 836 (38, 156); 3467 x 3467 208, 214 (14, 180); x 6587 356, 356 (26, 180); 1907 x 12000 357, 369
+// (12, 240); x 20000 605, 603 (20, 240).
+AttnSplit split_plan(int64_t q_len, int64_t k_len, int heads) {
+  const int64_t qb = max((q_len + 31) / 32, (int64_t)kWaves);
+  const int64_t groups = (heads * qb + kWaves - 1) / kWaves, ntiles = (k_len + kBK - 1) / kBK;
+  const int64_t cus = device_cus(), rest = groups % cus;
+  AttnSplit sp = {nullptr, (int)groups, 0, 0, 0};
+  if (rest == 0) return sp;
+  const int64_t s = cus / rest, idle = cus - s * rest;
+  const int64_t k = idle > 0 ? (rest + idle - 1) / idle : 0;
+  const int64_t part = max(k > 0 ? (ntiles * k + k * s) / (1 + k * s) : (ntiles + s - 1) / s, (int64_t)kSplitMinTiles);
+  const int64_t parts = (ntiles + part - 1) / part;
+  if (parts < 2 || (ntiles - part) * cus < 5 * cus + 26 * rest) return sp;
+  sp.full_groups = (int)(groups - rest);
+  sp.split_groups = (int)rest;
+  sp.parts = (int)parts;
+  sp.part_tiles = (int)part;
+  return sp;
+}
+
 }  // namespace
 
 // Tried and dropped (same inputs, cfg-4 joint shape): two query blocks per wave, pipelined inside
@@ -366,12 +486,24 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int 
 // accumulators pinned in a0..a127 by inline asm (no accumulator copies, no spills, bit-identical):
 // 3-5 % slower than this kernel -- half the LDS operand reads and a higher clock (2.1 against
 // 1.87 GHz), but the single wave's own latencies exposed (MFMA busy 0.47 against 0.55).
-hipError_t launch_attention_fwd(const AttnArgs& a, hipStream_t st) {
+int64_t attention_workspace_bytes(int64_t q_len, int64_t k_len, int heads) {
+  const AttnSplit sp = split_plan(q_len, k_len, heads);
+  return (int64_t)sp.split_groups * sp.parts * kPartSlot * (int64_t)sizeof(float);
+}
+
+hipError_t launch_attention_fwd(const AttnArgs& a, void* workspace, int64_t workspace_bytes, hipStream_t st) {
   // query blocks per head: at least kWaves, so a workgroup spans at most two heads
   const int qb = (int)max((a.q_len + 31) / 32, (int64_t)kWaves);
   const int64_t blocks = (int64_t)a.heads * qb;
-  const dim3 grid((unsigned)((blocks + kWaves - 1) / kWaves));
-  hipLaunchKernelGGL(attn_fwd_d128, grid, dim3(64 * kWaves), 0, st, a, qb);
+  AttnSplit sp = split_plan(a.q_len, a.k_len, a.heads);
+  if (sp.split_groups > 0 &&
+      (!workspace || workspace_bytes < (int64_t)sp.split_groups * sp.parts * kPartSlot * (int64_t)sizeof(float)))
+    sp = {nullptr, (int)((blocks + kWaves - 1) / kWaves), 0, 0, 0};
+  sp.ws = (float*)workspace;
+  hipLaunchKernelGGL(attn_fwd_d128, dim3((unsigned)(sp.full_groups + sp.split_groups * sp.parts)), dim3(64 * kWaves),
+                     0, st, a, qb, sp);
+  if (sp.split_groups > 0)
+    hipLaunchKernelGGL(attn_combine, dim3((unsigned)(sp.split_groups * kWaves)), dim3(256), 0, st, a, qb, sp);
   return hipGetLastError();
 }
 

@@ -636,9 +636,21 @@ joy_status joy_fused_cached_kv_pack(const joy_bf16_view* key0, const joy_bf16_vi
 }
 
 
+int64_t joy_attention_workspace_size(int64_t q_len, int64_t k_len, int64_t num_heads) {
+  if (q_len <= 0 || k_len <= 0 || num_heads <= 0 || num_heads > 65535) return 0;
+  if (num_heads * ((q_len + 31) / 32 + 8) > 0x7fffffffLL) return 0;
+  return joy::attention_workspace_bytes(q_len, k_len, (int)num_heads);
+}
+
 joy_status joy_attention_fwd(const joy_bf16_view* q, const joy_bf16_view* k, const joy_bf16_view* v, void* out,
                              int64_t out_stride_token, int64_t num_heads, int64_t head_dim, float scale,
                              void* stream) {
+  return joy_attention_fwd_workspace(q, k, v, out, out_stride_token, num_heads, head_dim, scale, nullptr, 0, stream);
+}
+
+joy_status joy_attention_fwd_workspace(const joy_bf16_view* q, const joy_bf16_view* k, const joy_bf16_view* v,
+                                       void* out, int64_t out_stride_token, int64_t num_heads, int64_t head_dim,
+                                       float scale, void* workspace, int64_t workspace_bytes, void* stream) {
   if (head_dim != 128) return fail(JOY_ERR_UNSUPPORTED, "attention_fwd supports head_dim=128 only");
   if (!q || !k || !v) return fail(JOY_ERR_INVALID_ARGUMENT, "q, k and v views must be non-null");
   if (q->len < 0 || k->len < 0 || v->len != k->len)
@@ -660,6 +672,7 @@ joy_status joy_attention_fwd(const joy_bf16_view* q, const joy_bf16_view* k, con
     return fail(JOY_ERR_UNSUPPORTED, "out needs 16-byte aligned rows");
   if (num_heads * ((q->len + 31) / 32 + 8) > 0x7fffffffLL)
     return fail(JOY_ERR_UNSUPPORTED, "num_heads * query blocks of 32 above 2^31");
+  if (workspace && !aligned(workspace, 16)) return fail(JOY_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
   joy::AttnArgs a;
   a.q = row_view(q);
   a.k = row_view(k);
@@ -670,7 +683,7 @@ joy_status joy_attention_fwd(const joy_bf16_view* q, const joy_bf16_view* k, con
   a.k_len = k->len;
   a.heads = (int)num_heads;
   a.scale_log2e = scale * 1.4426950408889634f;
-  return hip_status(joy::launch_attention_fwd(a, (hipStream_t)stream), "attention_fwd launch");
+  return hip_status(joy::launch_attention_fwd(a, workspace, workspace_bytes, (hipStream_t)stream), "attention_fwd launch");
 }
 
 }  // extern "C"

@@ -133,7 +133,10 @@ int64_t fp8_gemm_workspace_bytes(int M, int N, int K);
 hipError_t launch_norm_modulate(const NormModArgs& a, hipStream_t st);
 hipError_t launch_joint_qkv_pack(const JointPackArgs& a, hipStream_t st);
 hipError_t launch_cached_kv_pack(const CachedPackArgs& a, hipStream_t st);
-hipError_t launch_attention_fwd(const AttnArgs& a, hipStream_t st);
+// workspace (16-byte aligned) or null: used when workspace_bytes covers attention_workspace_bytes
+hipError_t launch_attention_fwd(const AttnArgs& a, void* workspace, int64_t workspace_bytes, hipStream_t st);
+// Workspace bytes the attention of this shape can use on the current device (0: none).
+int64_t attention_workspace_bytes(int64_t q_len, int64_t k_len, int heads);
 
 // Compute units of the current device, and workgroups of `threads` threads of `kern` that
 // stay resident per CU (HIP occupancy API, at least 1); both cached (device_info.hip).

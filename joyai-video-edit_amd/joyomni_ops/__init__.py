@@ -466,10 +466,15 @@ def _attention_impl(query, key, value, out, scale):
     B, Lq, H, D = _attention_checks(query, key, value, out)
     sc = float(scale) if scale is not None else 1.0 / math.sqrt(D)
     with torch.cuda.device(query.device):
+        # fp32 parts of the key split (0 bytes where the call is not split), shared by the batches,
+        # which follow each other on one stream
+        nbytes = _LIB.joy_attention_workspace_size(Lq, key.size(1), H) if D == 128 else 0
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes > 0 else None
         for b in range(B):
             qv, kv, vv = _view(query[b:b + 1]), _view(key[b:b + 1]), _view(value[b:b + 1])
-            st = _LIB.joy_attention_fwd(ctypes.byref(qv), ctypes.byref(kv), ctypes.byref(vv),
-                                        out[b].data_ptr(), out.stride(1), H, D, sc, _stream(query))
+            st = _LIB.joy_attention_fwd_workspace(ctypes.byref(qv), ctypes.byref(kv), ctypes.byref(vv),
+                                                  out[b].data_ptr(), out.stride(1), H, D, sc, _ptr(ws), nbytes,
+                                                  _stream(query))
             _lib.check(_LIB, st)
 
 

@@ -73,6 +73,8 @@ SIGNATURES = {
     "joy_fused_cached_kv_pack": (
         _int, [_view, _view, _view, _view, _vp, _vp, _i64, _i64, _vp, _vp, _vp]),
     "joy_attention_fwd": (_int, [_view, _view, _view, _vp, _i64, _i64, _i64, _f32, _vp]),
+    "joy_attention_workspace_size": (_i64, [_i64, _i64, _i64]),
+    "joy_attention_fwd_workspace": (_int, [_view, _view, _view, _vp, _i64, _i64, _i64, _f32, _vp, _i64, _vp]),
     "joy_fused_norm_scale_shift": (
         _int, [_vp, _i64, _int, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _int, _f32, _vp]),
     "joy_fused_norm_scale_shift_fp8": (
@@ -80,7 +82,7 @@ SIGNATURES = {
                _vp]),
 }
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 
 class JoyError(RuntimeError):

@@ -193,3 +193,79 @@ def test_reference_production_shape_sampled_queries(Lk):
     rows = np.sort(np.random.default_rng(Lk).choice(Lq, 48, replace=False))
     rows[0], rows[-1] = 0, Lq - 1
     _check(out, q, k, v, f"production {Lq}x{Lk}x{H}", rows=rows)
+
+
+def _split_call(q, k, v, workspace):
+    """joy_attention_fwd_workspace on [L, H, 128] device tensors, with its workspace or with none."""
+    import ctypes
+    import joyomni_ops as jo
+    from joyomni_ops import _lib
+    lib, H = jo._LIB, q.size(1)
+    view = lambda t: ctypes.byref(_lib.Bf16View(t.data_ptr(), t.size(0), t.stride(0), t.stride(1)))  # noqa: E731
+    nbytes = lib.joy_attention_workspace_size(q.size(0), k.size(0), H) if workspace else 0
+    ws = torch.full((nbytes + 64,), 0xff, dtype=torch.uint8, device=DEV)  # NaN where nothing is written
+    out = torch.full_like(q, float("nan"))
+    st = lib.joy_attention_fwd_workspace(view(q), view(k), view(v), out.data_ptr(), H * 128, H, 128,
+                                         1 / math.sqrt(128), ws.data_ptr(), nbytes,
+                                         torch.cuda.current_stream().cuda_stream)
+    _lib.check(lib, st)
+    torch.cuda.synchronize()
+    assert bool((ws[nbytes:] == 0xff).all())
+    return nbytes, out
+
+
+# few groups with many parts; parts and a shorter last one; a whole round before the split groups (257 and 264
+# groups on 256 CUs); a partial key tile alone in the last part, and none; padding blocks in the last group
+@pytest.mark.parametrize("Lq,Lk,H", [(1, 4001, 1), (100, 1600, 3), (512, 1025, 32), (859, 2001, 32), (65, 1152, 40),
+                                     (2056, 1400, 32), (2100, 2100, 32), (330, 3000, 7)])
+def test_key_split_matches_unsplit_and_oracle(Lq, Lk, H):
+    """The key split against the unsplit call: both round the probabilities to bf16 against their own
+    running max (2^-9 of a weight each) and the result to bf16 (2^-9), so each element is within 2^-7 of
+    max|v| + |ref| of the other; sampled rows against the oracle as everywhere."""
+    announce("attention key split", Lq, Lk, H)
+    q, k, v = _inputs(Lq, Lk, H, Lq * 7 + Lk)
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    none, whole = _split_call(qd, kd, vd, False)
+    nbytes, split = _split_call(qd, kd, vd, True)
+    assert none == 0 and nbytes > 0
+    vmax = vd.float().abs().amax(dim=(0, 2))[None, :, None]
+    assert bool(((split.float() - whole.float()).abs() <= 2.0 ** -7 * (vmax + whole.float().abs())).all())
+    rows = np.unique(np.random.default_rng(Lk).choice(Lq, min(Lq, 24)))
+    rows[-1] = Lq - 1
+    _check(split, q, k, v, f"split {Lq}x{Lk}x{H}", rows=rows)
+
+
+def test_key_split_with_parts_that_add_nothing():
+    """Keys of whole parts with scores of -inf (an infinite key component against positive queries) and
+    rising scores from part to part: the -inf keys weigh nothing, wherever the parts begin."""
+    announce("attention key split -inf")
+    Lq, Lk, H = 64, 2048, 4
+    q, k, v = _inputs(Lq, Lk, H, 5)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    k[:, :, 1] = (torch.arange(Lk) / 64)[:, None].to(torch.bfloat16)
+    k[: Lk // 4, :, 0] = float("-inf")
+    k[Lk // 2: Lk // 2 + 300, :, 0] = float("-inf")
+    nbytes, out = _split_call(q.to(DEV), k.to(DEV), v.to(DEV), True)
+    assert nbytes > 0
+    keep = torch.isfinite(k[:, 0, 0])
+    _check(out, q, k[keep], v[keep], "split -inf")
+
+
+def test_key_split_in_a_captured_graph():
+    """sdpa_attention with a split captured into a HIP graph and replayed with eager work between."""
+    announce("attention key split captured")
+    import joyomni_ops as jo
+    q, k, v = (t[None].to(DEV) for t in _inputs(512, 2000, 16, 6))
+    ref = jo.sdpa_attention(q, k, v)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            out = jo.sdpa_attention(q, k, v)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        jo.sdpa_attention(q.flip(1), v, k)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
