@@ -13,7 +13,7 @@
 // sgl_fused_ops.py:302-305); residual and output may be the same buffer.
 //
 // Kernels by problem shape:
-//  * fp8_gemm_4q (K % 256 == 0, M % 4 == 0, M > 512): persistent 256x256 tiles, one
+//  * fp8_gemm_4q (K % 256 == 0, M > 512): persistent 256x256 tiles, one
 //    workgroup per CU walking the whole rounds, 128-byte K steps through a 2-slot ring,
 //    16x16x128 MFMAs;
 //  * fp8_gemm_4k (M <= 512, and long-K GEMMs of less than one round): deep-K tiles
@@ -833,13 +833,17 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
     for (int i = 0; i < IW; ++i) dma_buf16(base + A_BYTES + (wave * IW + i) * 1024, ow[i], wrs, koff);
   };
   auto issue_side = [&](int mm, int nn) {
-    const int lr = min(lane, (M - mm) / 4 - 1), lc = min(lane, (N - nn) / 4 - 1), lb = min(lane, (N - nn) / 8 - 1);
-    const void* ps = sa + mm + 4 * lr;
+    const int lc = min(lane, (N - nn) / 4 - 1), lb = min(lane, (N - nn) / 8 - 1);
+    const void* ps = sa + min(mm + 4 * lane, M - 4);  // M > 4; rows past M - 4: see sa_index
     const void* pc = sb + nn + 4 * lc;
     const void* pb = has_bias ? (const void*)(bias + nn + 8 * lb) : pc;
     const void* src = wave == 0 ? ps : (wave == 2 ? pb : pc);
     dma_glb16(lds_u32((lds_void*)(side_lds + wave * 1024)), src);
   };
+
+  // where side_lds holds the scale of row r of the tile at row mm: lane r / 4 fetched the 4 scales from row
+  // 4 (r / 4) of the tile on, or the last 4 of all rows where those reach past M (any M, no load past it)
+  auto sa_index = [&](int r, int mm) { return r + max(0, (r & ~3) - (M - 4 - mm)); };
 
   v4f acc[FN][FM];
   v8i fw[FN], fa[FM];
@@ -1002,7 +1006,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
           asm volatile("v_mov_b32 %0, 0" : "=v"(jz));
           if (region < 2 && j + 1 < FM) load_tables(j + 1, tbn);
           // the GEMM's rounded output (as the plain epilogue stores it)
-          const float s_a = sa_l[wm * WTM + j * 16 + er];
+          const float s_a = sa_l[sa_index(wm * WTM + j * 16 + er, tm0)];
           uint2 yb[FN];
 #pragma unroll
           for (int i = 0; i < FN; ++i) {
@@ -1113,7 +1117,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
             rx[k] = __builtin_amdgcn_raw_buffer_load_b128(rrs, (int)roff, 0, 0);
           }
         }
-        const float s_a = sa_l[wm * WTM + j * 16 + er];
+        const float s_a = sa_l[sa_index(wm * WTM + j * 16 + er, tm0)];
         uint8_t* srow = stage + er * PITCH + eg * 8;
 #pragma unroll
         for (int i = 0; i < FN; ++i) {
@@ -1483,11 +1487,14 @@ ResidualArgs residual_args(const GemmArgs& g) {
 }
 
 
-// Layout rules of the persistent kernel fp8_gemm_4q: K steps in pairs of 128 bytes, row scales
-// read 4 at a time, 32-bit buffer offsets for the operands, the output and the residual.
+// Layout rules of the persistent kernel fp8_gemm_4q: K steps in pairs of 128 bytes, at least 4
+// rows (row scales are read 4 at a time), 32-bit buffer offsets for the operands, the output and
+// the residual. Row counts that are no multiple of 4 took the 64-byte-step kernel (and the fused
+// QKV projection its two-launch form): 3517 x 4096 -> 16384 with GELU 240 -> 207 us, 7019 x 16384
+// -> 4096 with the residual 433 -> 362, fused QKV 10797 x 5120 -> 15360 901 -> 702.
 bool persistent_ok(const GemmArgs& g) {
   constexpr int64_t kLim = 0x7fffffffLL;
-  return g.K % 256 == 0 && g.K >= 512 && g.M % 4 == 0 && (int64_t)g.M * g.K <= kLim && (int64_t)g.N * g.K <= kLim &&
+  return g.K % 256 == 0 && g.K >= 512 && g.M >= 4 && (int64_t)g.M * g.K <= kLim && (int64_t)g.N * g.K <= kLim &&
          ((int64_t)(g.M - 1) * g.ldc + g.N) * 2 <= kLim &&
          (!g.residual || ((int64_t)(g.M - 1) * g.ldr + g.N) * 2 <= kLim);
 }
@@ -1542,8 +1549,8 @@ hipError_t launch_4w(const GemmArgs& g, hipStream_t st) {
   constexpr int D = 5;  // DMA ring depth
   const int bulk = tiles_m * tiles_n - rem;
   // the persistent kernel takes the full rounds (or a single partial one) when its layout
-  // rules hold (K steps in pairs of 128 bytes, row scales read 4 at a time, 32-bit buffer
-  // offsets, a workgroup count that keeps the XCD mapping); with fewer tiles than CUs it
+  // rules hold (K steps in pairs of 128 bytes, 32-bit buffer offsets, a workgroup count that
+  // keeps the XCD mapping); with fewer tiles than CUs it
   // runs one tile per workgroup (1024 x 4096 -> 16384: 63 us vs 66 for the one-tile kernel,
   // 3120 x 4096 -> 4096: 53 vs 56, 1560 x 4096 -> 12288: 90 vs 95 with the sub-tile tail)
   bool persistent = false;

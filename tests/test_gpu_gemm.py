@@ -453,3 +453,40 @@ def test_persistent_rounds_match_per_tile_launch(M, kind):
         rows[-1] = M - 1
         assert_acc_bound(whole[rows], qa[rows], qw, sa[rows], sw, b if b is not None else np.zeros(N, np.uint16),
                          f"persistent {kind}")
+
+
+# rows past the last whole tile row: 1, 3 (fewer than one 4-row group), 2 and 255, beside whole rounds (4099: 17 x 16
+# tiles, the last one with 3 rows) and a 256x192 plan (1021)
+@pytest.mark.parametrize("kind", ["plain", "gelu", "residual"])
+@pytest.mark.parametrize("M,N,K", [(513, 520, 512), (1027, 264, 768), (4099, 4096, 512), (2303, 1032, 512),
+                                   (1021, 12288, 4096)])
+def test_persistent_kernel_any_row_count(M, N, K, kind):
+    """The persistent kernel with row counts that are no multiple of 4 and row scales that start 4 bytes past a
+    16-byte boundary: exact operands, so every row has its own scale and the output is fixed to the bit (GELU
+    against the oracle's own rounding of it, within one bf16 step)."""
+    announce("gemm odd rows", M, N, K, kind)
+    import joyomni_ops as jo
+    rng = np.random.default_rng(M + N)
+    qa = f32_to_e4m3fn(rng.integers(-8, 9, (M, K)).astype(np.float32))
+    qw = f32_to_e4m3fn(rng.integers(-8, 9, (N, K)).astype(np.float32))
+    sa = (2.0 ** rng.integers(-10, -5, M)).astype(np.float32)
+    sw = (2.0 ** rng.integers(-8, -4, N)).astype(np.float32)
+    bias = f32_to_bf16((rng.integers(-64, 64, N) / 16).astype(np.float32))
+    exp_bits, _ = og.scaled_mm(qa, qw, sa, sw, bias)
+    a, w = to_dev_fp8(qa), to_dev_fp8(qw).t()
+    sad = torch.empty(M + 1, device=DEV)[1:].copy_(torch.from_numpy(sa))
+    swd = torch.from_numpy(sw).to(DEV)
+    b = torch.from_numpy(bias.view(np.int16)).view(torch.bfloat16).to(DEV)
+    if kind == "plain":
+        assert np.array_equal(u16(jo.fp8_scaled_mm(a, w, sad, swd, torch.bfloat16, b)), exp_bits)
+    elif kind == "gelu":
+        got = bf16_to_f32(u16(jo.fp8_scaled_mm_gelu_tanh(a, w, sad, swd, torch.bfloat16, b)))
+        exp = torch.nn.functional.gelu(torch.from_numpy(bf16_to_f32(exp_bits)).double(), approximate="tanh").numpy()
+        assert (np.abs(got - exp) <= 2.0 ** -8 * np.abs(exp) + 1e-6).all()
+    else:
+        g = gen(M)
+        x, gate = torch.randn(M, N, generator=g).bfloat16(), torch.randn(N, generator=g).bfloat16()
+        y = torch.from_numpy(exp_bits.view(np.int16)).view(torch.bfloat16)
+        ref = torch.addcmul(x, y, gate)
+        got = jo.fp8_scaled_mm_gated_residual(a, w, sad, swd, x.to(DEV), gate.to(DEV), b)
+        assert torch.equal(got.cpu(), ref)

@@ -116,7 +116,7 @@ def u16_t(t):
     (777, 512, 5, 128),     # odd head count: fallback
     (300, 1024, 6, 64),     # head_dim 64: fallback
     (640, 640, 4, 128),     # K % 256 != 0: fallback
-    (1002, 1024, 8, 128),   # M % 4 != 0 (row scales read 4 at a time by the persistent kernel): fallback
+    (1002, 1024, 8, 128),   # M % 4 != 0
 ])
 def test_exact_equals_gemm_then_norm_rope(M, K, H, D):
     announce("fp8 qkv norm rope exact", M, K, H, D)
@@ -199,3 +199,9 @@ def test_no_ring_rows_written():
     """cache_tokens = 0: the ring keeps every row; Q / K / V are still written."""
     announce("fp8 qkv norm rope no ring rows")
     _run_both(4352, 1024, 32, 128, 15, exact=True, cache_tokens=0)
+
+
+@pytest.mark.parametrize("M", [515, 4353, 4354])  # a partial last tile row of 3, 1 and 2 rows
+def test_any_row_count(M):
+    """Token counts that are no multiple of 4 take the fused epilogue like the others."""
+    _run_both(M, 512, 4, 128, 90 + M, exact=True)
