@@ -1510,44 +1510,59 @@ hipError_t launch_one_round_256x128(const GemmArgs& g, int tm, int tn, hipStream
   return hipGetLastError();
 }
 
-// Full rounds of 256x256 tiles (one workgroup per CU), then the remaining tiles of
-// the last, partial round split into 4 (128x128) or 2 (256x128) sub-tiles so that
-// more CUs share that round. Both launches go to the same stream; the result does
-// not depend on the split (every output element sums its K products in the same order).
-template <bool kBf16, int kEpi>
-hipError_t launch_4w(const GemmArgs& g, hipStream_t st) {
-  int tiles_m = (g.M + 255) / 256;
-  const int tiles_n = (g.N + 255) / 256;
-  const int T = tiles_m * tiles_n, P = device_cus();
-  int rem = T % P;
-  int sub_log2 = 0;
-  if (rem * 4 <= P) {
-    sub_log2 = 2;
-  } else if (rem * 2 <= P + P / 4) {
-    sub_log2 = 1;
+// Tile plan of a GEMM of 256x256 tiles: `bulk` of them in whole rounds (one workgroup per CU), then
+// the rest of the last, partial round split into 4 (128x128, sub_log2 2) or 2 (256x128, sub_log2 1)
+// sub-tiles so that more CUs share that round (not split where it is nearly full), or, with a short
+// last tile row, sub_log2 -4 (decode_job). The plain, GELU and residual GEMMs and the fused QKV
+// projection share it; the result does not depend on the split (every output element sums its K
+// products in the same order).
+struct TilePlan {
+  int tiles_m, tiles_n, bulk, rem, sub_log2;
+};
+TilePlan tile_plan(int M, int N, int K) {
+  TilePlan p;
+  p.tiles_m = (M + 255) / 256;
+  p.tiles_n = (N + 255) / 256;
+  const int T = p.tiles_m * p.tiles_n, P = device_cus();
+  p.rem = T % P;
+  p.sub_log2 = 0;
+  if (p.rem * 4 <= P) {
+    p.sub_log2 = 2;
+  } else if (p.rem * 2 <= P + P / 4) {
+    p.sub_log2 = 1;
   } else {
-    rem = 0;  // the last round is nearly full: no split
+    p.rem = 0;  // the last round is nearly full: no split
   }
   // With at most 128 rows in the last tile row, its 256x256 tiles are mostly padding: when the
   // whole tile rows' leftover tiles (as 128x128 quarters) and the last row's top halves (one
   // 128x128 tile per 128 columns) fit one round, that round takes a quarter tile's time instead
   // of a half (1560 x 4096 -> 12288: one round of 256 tiles, then 32 x 4 + 96 = 224 quarter tiles
   // instead of 80 x 2 half tiles)
-  bool last_row_quarters = false;
-  const int m_rows = g.M % 256;
-  if (m_rows > 0 && m_rows <= 128 && g.M > 256 && g.K % 128 == 0) {
-    const int tf = (g.M / 256) * tiles_n;
-    const int lq = (tf % P) * 4 + (g.N + 127) / 128;
-    const int cost_now = 4 * (T / P) + (rem == 0 ? 4 * ((T % P) != 0) : (sub_log2 == 2 ? 1 : 2));
-    if (tf >= P && lq <= P && 4 * (tf / P) + 1 < cost_now) last_row_quarters = true;
+  const int m_rows = M % 256;
+  if (m_rows > 0 && m_rows <= 128 && M > 256 && K % 128 == 0) {
+    const int tf = (M / 256) * p.tiles_n;
+    const int lq = (tf % P) * 4 + (N + 127) / 128;
+    const int cost_now = 4 * (T / P) + (p.rem == 0 ? 4 * ((T % P) != 0) : (p.sub_log2 == 2 ? 1 : 2));
+    if (tf >= P && lq <= P && 4 * (tf / P) + 1 < cost_now) {
+      p.tiles_m = M / 256;
+      p.rem = tf % P;
+      p.sub_log2 = -4;
+    }
   }
-  if (last_row_quarters) {
-    tiles_m = g.M / 256;
-    rem = (tiles_m * tiles_n) % P;
-    sub_log2 = -4;
-  }
+  p.bulk = p.tiles_m * p.tiles_n - p.rem;
+  return p;
+}
+// 128x128 sub-tiles of a plan's last launch with sub_log2 -4: four per leftover tile, one per 128
+// columns of the short last tile row
+int quarter_tiles(const TilePlan& p, int N) { return p.rem * 4 + (N + 127) / 128; }
+
+// The tile plan's launches, on the same stream.
+template <bool kBf16, int kEpi>
+hipError_t launch_4w(const GemmArgs& g, hipStream_t st) {
+  const int P = device_cus();
+  const TilePlan tp = tile_plan(g.M, g.N, g.K);
+  const int tiles_m = tp.tiles_m, tiles_n = tp.tiles_n, bulk = tp.bulk, rem = tp.rem, sub_log2 = tp.sub_log2;
   constexpr int D = 5;  // DMA ring depth
-  const int bulk = tiles_m * tiles_n - rem;
   // the persistent kernel takes the full rounds (or a single partial one) when its layout
   // rules hold (K steps in pairs of 128 bytes, 32-bit buffer offsets, a workgroup count that
   // keeps the XCD mapping); with fewer tiles than CUs it
@@ -1567,10 +1582,9 @@ hipError_t launch_4w(const GemmArgs& g, hipStream_t st) {
                        g.scales_b, (const uint16_t*)g.bias, (uint16_t*)g.C, g.M, g.N, g.K, g.ldc, tiles_m, tiles_n,
                        kGroupM, 0, -1, residual_args(g), nullptr, 1);
   }
-  if (last_row_quarters) {
-    const int nq = rem * 4 + (g.N + 127) / 128;
-    hipLaunchKernelGGL((fp8_gemm_4h<kBf16, kEpi, 128, 128, 4>), dim3(nq), dim3(256), 0, st, (const uint8_t*)g.A,
-                       (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias, (uint16_t*)g.C, g.M, g.N,
+  if (sub_log2 == -4) {
+    hipLaunchKernelGGL((fp8_gemm_4h<kBf16, kEpi, 128, 128, 4>), dim3(quarter_tiles(tp, g.N)), dim3(256), 0, st,
+                       (const uint8_t*)g.A, (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias, (uint16_t*)g.C, g.M, g.N,
                        g.K, g.ldc, tiles_m, tiles_n, kGroupM, bulk, -4, residual_args(g));
   } else if (rem > 0) {
     if (sub_log2 == 2) {
@@ -2046,17 +2060,36 @@ hipError_t launch_gemm_t(const GemmArgs& g, hipStream_t st) {
 }
 
 // q/k RMSNorm + RoPE and the KV-ring write of the tiles of a fused QKV projection that the
-// persistent kernel leaves to the sub-tile launch (which stores them plainly in C): one
-// workgroup per sub-tile of BMs rows x one head, 16 lanes per token as in the standalone
-// kernel (same arithmetic order, head_rsqrt), the sub-tile order of fp8_gemm_4h.
+// persistent kernel leaves to the sub-tile launch (which stores them plainly in C): 16 lanes per
+// token's head as in the standalone kernel (same arithmetic order, head_rsqrt), the sub-tile order
+// of fp8_gemm_4h in blockIdx.x, kTailRows of the sub-tile's BMs rows in blockIdx.y. Memory-bound
+// (20 to 40 MB), so it wants loads in flight: a workgroup that walked a whole sub-tile, 16 rows at
+// a time, left 160 to 256 workgroups with one load each in flight: the whole op at 1560 x 4096 ->
+// 12288 109.5 -> 91.0 us (with the tile plan's quarter tiles for its 24-row last tile row), at
+// 3120 rows 163.9 -> 154.6, at 300 rows 49.3 -> 37.0, at 10800 x 5120 -> 15360 710 -> 695.
+constexpr int kTailRows = 32;
 template <int BMs>
 __global__ __launch_bounds__(256) void qkv_tail_norm_rope(const uint16_t* __restrict__ C, int64_t ldc, int M,
                                                           int tiles_m, int tiles_n, int group_m, int tile_base,
                                                           int sub_log2, QkvEpi qe) {
   const TileJob job = decode_job<BMs, 128>(0, tiles_m, tiles_n, group_m, tile_base, sub_log2, 1);
+  const int row0 = job.m0 + (int)blockIdx.y * kTailRows;
+  if (row0 >= M) return;
   const int lane = threadIdx.x & 63, li = lane & 15;
   const int eh = qe.heads * 128, region = job.n0 / eh, head = (job.n0 - region * eh) >> 7;
   const int o1 = region == 0 ? 0 : (region == 1 ? 1 : 3), o2 = region == 1 ? 2 : 4;
+  constexpr int U = kTailRows / 16;
+  uint4 x[U];
+  uint2 cv[U], sv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int mr = min(row0 + u * 16 + (int)(threadIdx.x >> 4), M - 1);  // every lane takes part in the shuffles
+    x[u] = *(const uint4*)(C + (int64_t)mr * ldc + job.n0 + li * 8);
+    if (region < 2) {
+      cv[u] = *(const uint2*)(qe.cos + (int64_t)mr * 64 + li * 4);
+      sv[u] = *(const uint2*)(qe.sin + (int64_t)mr * 64 + li * 4);
+    }
+  }
   float w[8] = {};
   if (region < 2) {
     const uint4 wv = *(const uint4*)((region == 0 ? qe.q_weight : qe.k_weight) + li * 8);
@@ -2067,13 +2100,12 @@ __global__ __launch_bounds__(256) void qkv_tail_norm_rope(const uint16_t* __rest
       w[2 * e + 1] = bf16_hi(ww[e]);
     }
   }
-  for (int u0 = 0; u0 < BMs; u0 += 16) {
-    const int m = job.m0 + u0 + (int)(threadIdx.x >> 4);
-    const int mr = min(m, M - 1);  // every lane takes part in the head's shuffles
-    const uint4 x = *(const uint4*)(C + (int64_t)mr * ldc + job.n0 + li * 8);
-    uint4 out1 = x, out2 = x;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int m = row0 + u * 16 + (int)(threadIdx.x >> 4);
+    uint4 out1 = x[u], out2 = x[u];
     if (region < 2) {
-      const uint32_t xw[4] = {x.x, x.y, x.z, x.w};
+      const uint32_t xw[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
       float f[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -2088,10 +2120,8 @@ __global__ __launch_bounds__(256) void qkv_tail_norm_rope(const uint16_t* __rest
       const float r = head_rsqrt(ss, 1.0f / 128.0f, qe.eps);
 #pragma unroll
       for (int j = 0; j < 8; ++j) f[j] = f[j] * r * w[j];
-      const uint2 cv = *(const uint2*)(qe.cos + (int64_t)mr * 64 + li * 4);
-      const uint2 sv = *(const uint2*)(qe.sin + (int64_t)mr * 64 + li * 4);
-      const float c[4] = {bf16_lo(cv.x), bf16_hi(cv.x), bf16_lo(cv.y), bf16_hi(cv.y)};
-      const float sn[4] = {bf16_lo(sv.x), bf16_hi(sv.x), bf16_lo(sv.y), bf16_hi(sv.y)};
+      const float c[4] = {bf16_lo(cv[u].x), bf16_hi(cv[u].x), bf16_lo(cv[u].y), bf16_hi(cv[u].y)};
+      const float sn[4] = {bf16_lo(sv[u].x), bf16_hi(sv[u].x), bf16_lo(sv[u].y), bf16_hi(sv[u].y)};
       float o[8];
 #pragma unroll
       for (int p = 0; p < 4; ++p) rope_pair(f[2 * p], f[2 * p + 1], c[p], sn[p], o[2 * p], o[2 * p + 1]);
@@ -2119,30 +2149,6 @@ int64_t fp8_gemm_workspace_bytes(int M, int N, int K) {
 }
 
 namespace {
-// Tile plan of the fused QKV projection: the persistent kernel takes the whole rounds of 256x256
-// tiles (or all tiles when the last round is nearly full), the rest run as 128x128 (sub 2) or
-// 256x128 (sub 1) sub-tiles, as launch_4w splits them.
-struct QkvPlan {
-  int tiles_m, tiles_n, bulk, rem, sub_log2;
-};
-QkvPlan qkv_plan(int M, int N) {
-  QkvPlan p;
-  p.tiles_m = (M + 255) / 256;
-  p.tiles_n = N / 256;
-  const int T = p.tiles_m * p.tiles_n, P = device_cus();
-  p.rem = T % P;
-  p.sub_log2 = 0;
-  if (p.rem * 4 <= P) {
-    p.sub_log2 = 2;
-  } else if (p.rem * 2 <= P + P / 4) {
-    p.sub_log2 = 1;
-  } else {
-    p.rem = 0;
-  }
-  p.bulk = T - p.rem;
-  return p;
-}
-
 bool qkv_fusable(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
   const int64_t eh = (int64_t)a.num_heads * 128;
   if (head_dim != 128 || !g.out_bf16 || g.gelu || g.residual || a.num_heads % 2 != 0 || g.N != 3 * eh) return false;
@@ -2154,6 +2160,13 @@ bool qkv_fusable(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
   return true;
 }
 }  // namespace
+
+// Whether some tiles of the fused QKV projection go through the scratch: the persistent kernel's
+// epilogue takes the whole rounds, the tail kernel the sub-tiles of the last, partial one.
+static bool qkv_has_tail(int M, int N, int K) {
+  const TilePlan p = tile_plan(M, N, K);
+  return p.rem > 0 || p.sub_log2 == -4;
+}
 
 int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_dim) {
   if (M <= 0 || N <= 0) return 0;
@@ -2167,19 +2180,19 @@ int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_
   a.num_heads = num_heads;
   a.n_tokens = a.table_len = M;
   a.q_out_stride = a.k_out_stride = a.kpre_stride = a.v_out_stride = a.v_out2_stride = (int64_t)num_heads * head_dim;
-  if (qkv_fusable(g, a, head_dim) && qkv_plan(M, N).rem == 0) return 0;
+  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(M, N, K)) return 0;
   return (int64_t)M * N * 2;
 }
 
 int64_t fp8_gemm_qkv_call_scratch_bytes(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
   if (g.M <= 0 || g.N <= 0) return 0;
-  if (qkv_fusable(g, a, head_dim) && qkv_plan(g.M, g.N).rem == 0) return 0;
+  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(g.M, g.N, g.K)) return 0;
   return (int64_t)g.M * g.N * 2;
 }
 
 hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int head_dim, hipStream_t st) {
   if (g.M == 0 || g.N == 0) return hipSuccess;
-  if (!qkv_fusable(g, a, head_dim) || (qkv_plan(g.M, g.N).rem > 0 && g.C == nullptr)) {
+  if (!qkv_fusable(g, a, head_dim) || (qkv_has_tail(g.M, g.N, g.K) && g.C == nullptr)) {
     // the GEMM into C, then the standalone norm/RoPE kernel on it
     if (g.C == nullptr) return hipErrorInvalidValue;
     hipError_t e = launch_fp8_gemm(g, st);
@@ -2211,7 +2224,7 @@ hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int hea
   qe.heads = a.num_heads;
   qe.eps = a.eps;
   qe.kpre_rotated = a.cache_post_rope;
-  const QkvPlan p = qkv_plan(g.M, g.N);
+  const TilePlan p = tile_plan(g.M, g.N, g.K);
   const int P = device_cus();
   if (p.bulk > 0) {
     hipLaunchKernelGGL((fp8_gemm_4q<true, kEpiQkv, 256>), dim3(p.bulk < P ? p.bulk : P), dim3(256), 0, st,
@@ -2221,20 +2234,21 @@ hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int hea
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (p.rem == 0) return hipSuccess;
+  if (!qkv_has_tail(g.M, g.N, g.K)) return hipSuccess;
   const uint16_t* c = (const uint16_t*)g.C;
-  if (p.sub_log2 == 2) {
-    hipLaunchKernelGGL((fp8_gemm_4h<true, kEpiPlain, 128, 128, 4>), dim3(p.rem << 2), dim3(256), 0, st,
-                       (const uint8_t*)g.A, (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias,
-                       (uint16_t*)g.C, g.M, g.N, g.K, g.ldc, p.tiles_m, p.tiles_n, kGroupM, p.bulk, 2, residual_args(g));
-    hipLaunchKernelGGL((qkv_tail_norm_rope<128>), dim3(p.rem << 2), dim3(256), 0, st, c, g.ldc, g.M, p.tiles_m,
-                       p.tiles_n, kGroupM, p.bulk, 2, qe);
-  } else {
+  if (p.sub_log2 == 1) {
     hipLaunchKernelGGL((fp8_gemm_4h<true, kEpiPlain, 256, 128, 3>), dim3(p.rem << 1), dim3(256), 0, st,
                        (const uint8_t*)g.A, (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias,
                        (uint16_t*)g.C, g.M, g.N, g.K, g.ldc, p.tiles_m, p.tiles_n, kGroupM, p.bulk, 1, residual_args(g));
-    hipLaunchKernelGGL((qkv_tail_norm_rope<256>), dim3(p.rem << 1), dim3(256), 0, st, c, g.ldc, g.M, p.tiles_m,
-                       p.tiles_n, kGroupM, p.bulk, 1, qe);
+    hipLaunchKernelGGL((qkv_tail_norm_rope<256>), dim3(p.rem << 1, 256 / kTailRows), dim3(256), 0, st, c, g.ldc, g.M,
+                       p.tiles_m, p.tiles_n, kGroupM, p.bulk, 1, qe);
+  } else {
+    const int n = p.sub_log2 == -4 ? quarter_tiles(p, g.N) : p.rem << 2;
+    hipLaunchKernelGGL((fp8_gemm_4h<true, kEpiPlain, 128, 128, 4>), dim3(n), dim3(256), 0, st, (const uint8_t*)g.A,
+                       (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias, (uint16_t*)g.C, g.M, g.N,
+                       g.K, g.ldc, p.tiles_m, p.tiles_n, kGroupM, p.bulk, p.sub_log2, residual_args(g));
+    hipLaunchKernelGGL((qkv_tail_norm_rope<128>), dim3(n, 128 / kTailRows), dim3(256), 0, st, c, g.ldc, g.M, p.tiles_m,
+                       p.tiles_n, kGroupM, p.bulk, p.sub_log2, qe);
   }
   return hipGetLastError();
 }
