@@ -10,6 +10,8 @@ import os
 
 LIB_NAME = "libjoyomni_hip.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
+# the operators' device implementations (csrc/torch_ops.cpp), linked to LIB_NAME beside it
+TORCH_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), "libjoyomni_torch.so")
 
 JOY_OK = 0
 JOY_ERR_INVALID_ARGUMENT = 1
@@ -102,6 +104,18 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     if lib.joy_abi_version() != ABI_VERSION:
         raise ImportError(f"{LIB_NAME} ABI version {lib.joy_abi_version()} != {ABI_VERSION}")
     return lib
+
+
+def load_ops() -> None:
+    """Register the operators' device implementations with torch."""
+    import torch
+    if not os.path.exists(TORCH_LIB_PATH):
+        raise ImportError(f"{os.path.basename(TORCH_LIB_PATH)} not found beside {LIB_NAME}; build it first "
+                          "(make -C joyai-video-edit_amd/csrc)")
+    try:
+        torch.ops.load_library(TORCH_LIB_PATH)
+    except OSError as e:
+        raise ImportError(str(e)) from e
 
 
 def check(lib: ctypes.CDLL, status: int) -> None:
