@@ -18,11 +18,10 @@
 //    16x16x128 MFMAs;
 //  * fp8_gemm_4k (M <= 512, and long-K GEMMs of less than one round): deep-K tiles
 //    with register-staged operands and optional split-K;
-//  * fp8_gemm_4n (129-512 rows with N % 80 == 0, e.g. N 5120): one round of narrow
-//    BM x 80 tiles, no K split;
+//  * fp8_gemm_4n (up to 512 rows, K < 8192): one round of narrow BM x BN tiles, no K split;
 //  * fp8_gemm_4h (K % 128 == 0): one 256x128 or 128x128 tile per workgroup with the
 //    persistent kernel's 128-byte K steps; the sub-tiles of the last, partial round and
-//    single-round GEMMs of <= 2048 rows that 256x128 tiles fill best;
+//    single-round GEMMs of <= 2048 rows;
 //  * fp8_gemm_4w (any M, N with K % 64 == 0): one tile per workgroup; the sub-tiles of
 //    the last, partial round when K % 128 != 0 and the remaining shapes. Its layout:
 //  * 256 threads = 4 waves in 2x2, one wave per SIMD; macro tile 256x256 (one workgroup
@@ -757,6 +756,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
   static_assert(kEpi == kEpiPlain || kEpi == kEpiGelu || kEpi == kEpiResidual || kEpi == kEpiQkv, "epilogues");
   static_assert(kEpi != kEpiQkv || (BN == 256 && kBf16), "fused QKV epilogue: 256-wide tiles (one head per wave), bf16");
   static_assert(BN == 128 || BN == 192 || BN == 256, "tile widths");
+  constexpr bool kCopyScales = kEpi == kEpiPlain || kEpi == kEpiGelu;
   constexpr int BM = 256, KS = 128, NW = 4, S = 2;
   constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16, FH = FN / 2;
   constexpr int CPR = KS / 16, RPL = 64 / CPR;  // 8 chunks per row, 8 rows per DMA instruction
@@ -834,16 +834,14 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
   };
   auto issue_side = [&](int mm, int nn) {
     const int lc = min(lane, (N - nn) / 4 - 1), lb = min(lane, (N - nn) / 8 - 1);
-    const void* ps = sa + min(mm + 4 * lane, M - 4);  // M > 4; rows past M - 4: see sa_index
+    // row scales, 4 a lane, none past M (M >= 4): whole groups only, and the last 4 of all rows to wave 3's
+    // words (kCopyScales), or the last 4 in the last lane
+    const void* ps = sa + (kCopyScales ? mm + 4 * min(lane, (M - mm) / 4 - 1) : min(mm + 4 * lane, M - 4));
     const void* pc = sb + nn + 4 * lc;
     const void* pb = has_bias ? (const void*)(bias + nn + 8 * lb) : pc;
-    const void* src = wave == 0 ? ps : (wave == 2 ? pb : pc);
+    const void* src = wave == 0 ? ps : (wave == 2 ? pb : (kCopyScales && wave == 3 ? (const void*)(sa + M - 4) : pc));
     dma_glb16(lds_u32((lds_void*)(side_lds + wave * 1024)), src);
   };
-
-  // where side_lds holds the scale of row r of the tile at row mm: lane r / 4 fetched the 4 scales from row
-  // 4 (r / 4) of the tile on, or the last 4 of all rows where those reach past M (any M, no load past it)
-  auto sa_index = [&](int r, int mm) { return r + max(0, (r & ~3) - (M - 4 - mm)); };
 
   v4f acc[FN][FM];
   v8i fw[FN], fa[FM];
@@ -955,6 +953,19 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
       const uint16_t* bias_l = (const uint16_t*)(side_lds + 2048);
       uint8_t* stage = stage_lds + wave * STAGE;
       const int mw = tm0 + wm * WTM, nw0 = tn0 + wn * WTN;
+      // In the last tile row the last M % 4 row scales are not in their place (issue_side). Plain and
+      // GELU epilogues copy them there from wave 3's words, which hold the last 4: every wave
+      // writes the same values, before its own reads of them, and the other lanes copy an unused word
+      // onto itself (a branch costs the K loop 52 bytes of spills). The others, whose registers that
+      // would spill, find them 4 - M % 4 words further on (1-2 % slower in the first two).
+      if constexpr (kCopyScales) {
+        float* side = (float*)side_lds;
+        const int odd = tm0 + BM > M ? (M & 3) : 0;
+        const bool mine = lane_e < odd;
+        side[mine ? (M & 252) + lane_e : 832 + lane_e] = side[mine ? 772 - odd + lane_e : 832 + lane_e];
+        asm volatile("" ::: "memory");
+      }
+      auto row_scale = [&](int r) { return sa_l[kCopyScales ? r : r + max(0, (r & ~3) - (M - 4 - tm0))]; };
       typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
       if constexpr (kEpi == kEpiQkv) {
         // this wave's 128 columns are one head of q, k or v (the three blocks are 256-aligned)
@@ -1006,7 +1017,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
           asm volatile("v_mov_b32 %0, 0" : "=v"(jz));
           if (region < 2 && j + 1 < FM) load_tables(j + 1, tbn);
           // the GEMM's rounded output (as the plain epilogue stores it)
-          const float s_a = sa_l[sa_index(wm * WTM + j * 16 + er, tm0)];
+          const float s_a = row_scale(wm * WTM + j * 16 + er);
           uint2 yb[FN];
 #pragma unroll
           for (int i = 0; i < FN; ++i) {
@@ -1117,7 +1128,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
             rx[k] = __builtin_amdgcn_raw_buffer_load_b128(rrs, (int)roff, 0, 0);
           }
         }
-        const float s_a = sa_l[sa_index(wm * WTM + j * 16 + er, tm0)];
+        const float s_a = row_scale(wm * WTM + j * 16 + er);
         uint8_t* srow = stage + er * PITCH + eg * 8;
 #pragma unroll
         for (int i = 0; i < FN; ++i) {
@@ -1487,9 +1498,9 @@ ResidualArgs residual_args(const GemmArgs& g) {
 }
 
 
-// Layout rules of the persistent kernel fp8_gemm_4q: K steps in pairs of 128 bytes, at least 4
-// rows (row scales are read 4 at a time), 32-bit buffer offsets for the operands, the output and
-// the residual. Row counts that are no multiple of 4 took the 64-byte-step kernel (and the fused
+// Layout rules of the persistent kernel fp8_gemm_4q: K steps in pairs of 128 bytes, at least 4 rows,
+// 32-bit buffer offsets for the operands, the output and the residual. While it took multiples of 4
+// rows only (row scales are loaded 4 at a time), the others took the 64-byte-step kernel (and the fused
 // QKV projection its two-launch form): 3517 x 4096 -> 16384 with GELU 240 -> 207 us, 7019 x 16384
 // -> 4096 with the residual 433 -> 362, fused QKV 10797 x 5120 -> 15360 901 -> 702.
 bool persistent_ok(const GemmArgs& g) {
@@ -1499,15 +1510,39 @@ bool persistent_ok(const GemmArgs& g) {
          (!g.residual || ((int64_t)(g.M - 1) * g.ldr + g.N) * 2 <= kLim);
 }
 
-// One round of 256x128 tiles (tm x tn <= CUs), one tile per workgroup. The one-tile kernel's
-// 3-slot ring beats the persistent 16x16x128 kernel here (1560 x 4096 -> 4096: 29.0 vs 30.0 us,
-// 512 x 5120 -> 13824: 34.9 vs 38.9; same-process A/B, bit-identical).
-template <bool kBf16, int kEpi>
-hipError_t launch_one_round_256x128(const GemmArgs& g, int tm, int tn, hipStream_t st) {
-  hipLaunchKernelGGL((fp8_gemm_4h<kBf16, kEpi, 256, 128, 3>), dim3(tm * tn), dim3(256), 0, st, (const uint8_t*)g.A,
+// One round of one-tile workgroups with 128-byte K steps (fp8_gemm_4h): the smallest tile whose tiles
+// fit the CUs, if there are at least `least_tiles` of them; hipErrorNotFound where none does. Against
+// the register-staged deep-K kernel with the same tiles: 600 x 4096 -> 4096 18.8 -> 16.4 us, 1024 x 4096
+// -> 4096 21.4 -> 19.4, 800 x 16384 -> 4096 67.7 -> 62.3 (1024 rows: level); 192x128 tiles where 128x128
+// take more than a round: 800 x 5120 -> 5120 33.3 -> 27.8, 1024 x 5120 -> 5120 41.7 -> 30.2; 128x256:
+// 600 x 4096 -> 12288 37.7 -> 33.9. The 3-slot ring of 256x128 tiles also beats the persistent
+// 16x16x128 kernel here (1560 x 4096 -> 4096: 29.0 vs 30.0 us; bit-identical).
+template <bool kBf16, int kEpi, int BM, int BN, int S>
+hipError_t launch_4h(const GemmArgs& g, hipStream_t st) {
+  const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
+  hipLaunchKernelGGL((fp8_gemm_4h<kBf16, kEpi, BM, BN, S>), dim3(tm * tn), dim3(256), 0, st, (const uint8_t*)g.A,
                      (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias, (uint16_t*)g.C, g.M, g.N,
                      g.K, g.ldc, tm, tn, 1, 0, -2, residual_args(g));
   return hipGetLastError();
+}
+struct TileShape {
+  int bm, bn;
+};
+TileShape one_round_shape(int M, int N, int64_t least_tiles) {
+  constexpr TileShape kShapes[] = {{128, 128}, {192, 128}, {256, 128}, {128, 256}};  // in the order of area
+  for (const TileShape& s : kShapes) {
+    const int64_t t = (int64_t)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+    if (t <= device_cus() && t >= least_tiles) return s;
+  }
+  return {0, 0};
+}
+template <bool kBf16, int kEpi>
+hipError_t launch_one_round(const GemmArgs& g, int64_t least_tiles, hipStream_t st) {
+  const TileShape s = one_round_shape(g.M, g.N, least_tiles);
+  if (s.bm == 192) return launch_4h<kBf16, kEpi, 192, 128, 3>(g, st);
+  if (s.bm == 256) return launch_4h<kBf16, kEpi, 256, 128, 3>(g, st);
+  if (s.bm == 128) return s.bn == 128 ? launch_4h<kBf16, kEpi, 128, 128, 4>(g, st) : launch_4h<kBf16, kEpi, 128, 256, 3>(g, st);
+  return hipErrorNotFound;
 }
 
 // Tile plan of a GEMM of 256x256 tiles: `bulk` of them in whole rounds (one workgroup per CU), then
@@ -1708,16 +1743,15 @@ hipError_t launch_deepk(const GemmArgs& g, int splits, float* ws, hipStream_t st
 }
 
 // ---------------------------------------------------------------------------
-// Narrow tiles for small M with N % 80 == 0 (the model's 5120-wide outputs at 129-512 tokens):
-// BM x 80 tiles, BM = 64 or 128, so that one round of tiles fills the CUs without a K split
-// (M 256 x N 5120: 4 x 64 tiles of 64 x 80; M 512: 4 x 64 of 128 x 80). These GEMMs are bound by
-// the operand bytes each CU streams, (BM + BN) x K per tile, at 40-50 GB/s per CU when the
-// operands come partly from HBM (a load-only probe of the same access pattern takes 18.8 us at
-// M 512 x N 5120 with 128 x 80 tiles against 25.1 us with 128 x 128 tiles on 160 CUs, and
-// 14.7 us at M 256 with 64 x 80 tiles); of the tile shapes that fill one round, the squarest
-// moves the fewest bytes per CU.
+// Narrow tiles for small M (16-512 tokens: the condition stream, small chunks): BM x BN tiles, BM = 64
+// or 128, so that one round of tiles fills the CUs without a K split (narrow_plan). These GEMMs are
+// bound by the operand bytes each CU streams, (BM + BN) x K per tile, at 40-80 GB/s per CU when the
+// operands come partly from HBM: a copy of the one-tile DMA kernel without its MFMAs and LDS reads
+// takes 27.6 of 28.9 us at M 347 x N 16384 x K 4096, and three or four steps in flight instead of two,
+// or K orders that differ from panel to panel, change nothing. So the shape that fills one round
+// with the fewest BM + BN is the fastest.
 //
-// 4 x KH waves: wave w owns rows [(w % 4) BM/4, +BM/4) and all 80 columns, as FM x 5 tiles of
+// 4 x KH waves: wave w owns rows [(w % 4) BM/4, +BM/4) and all BN columns, as FM x FN tiles of
 // v_mfma_scale_f32_16x16x128_f8f6f4 (operand lanes and accumulator layout as in fp8_gemm_4q:
 // lane l holds row l % 16 of a fragment, K bytes [32 (l / 16), +32) of a 128-byte k-step;
 // accumulator element e of lane l is output (row l % 16, column 4 (l / 16) + e)). K steps of
@@ -1730,7 +1764,8 @@ hipError_t launch_deepk(const GemmArgs& g, int splits, float* ws, hipStream_t st
 // Workgroup positions are XCD-ordered with the tile rows innermost, so the tiles that share
 // a W panel run on one XCD and read it through one L2.
 // ---------------------------------------------------------------------------
-template <bool kBf16, int kEpi, int BM, int U, int KH>
+constexpr bool narrow_ragged(int bn) { return bn % 48 == 0; }
+template <bool kBf16, int kEpi, int BM, int BN, int U, int KH>
 __global__ __launch_bounds__(256 * KH, 1) void fp8_gemm_4n(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ W, const float* __restrict__ sa,
     const float* __restrict__ sb, const uint16_t* __restrict__ bias, uint16_t* __restrict__ C,
@@ -1739,13 +1774,14 @@ __global__ __launch_bounds__(256 * KH, 1) void fp8_gemm_4n(
   static_assert(U == 2 || U == 3, "staging buffers");
   static_assert(KH == 1 || KH == 2, "waves per row group");
   constexpr int UNR = U == 2 ? 2 : 6;  // lcm(U, 2 slots)
-  constexpr int BN = 80, KS = 256, NW = 4, NT = 256 * KH;
+  constexpr int KS = 256, NW = 4, NT = 256 * KH;
   constexpr int WTM = BM / NW, FM = WTM / 16, FN = BN / 16;
   constexpr int CPR = KS / 16;                                 // 16 chunks per row
   constexpr int ROWS = BM + BN, CHUNKS = ROWS * CPR;
   constexpr int L = (CHUNKS + NT - 1) / NT, LAST = CHUNKS - (L - 1) * NT;  // loads per thread; the last
   constexpr int SLOT = ROWS * KS, A_BYTES = BM * KS;                         // one by the first LAST threads
-  static_assert(BM == 64 || BM == 128, "tile heights");
+  static_assert(BM % 64 == 0 && BN % 16 == 0, "tile shapes");
+  constexpr bool kRagged = narrow_ragged(BN);  // whether the last column tile may reach past N
   static_assert(LAST % 64 == 0 && (NT / CPR) % 16 == 0 && BM % (NT / CPR) == 0, "whole waves per load, A or W rows");
   static_assert(2 * SLOT <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * SLOT];
@@ -1765,7 +1801,10 @@ __global__ __launch_bounds__(256 * KH, 1) void fp8_gemm_4n(
   for (int i = 0; i < L; ++i) {
     const int row = min(i * (NT / CPR) + tid / CPR, ROWS - 1);
     const int chunk = (lc ^ swz_rows<KS>(row)) * 16;
-    src[i] = row < BM ? A + (int64_t)min(m0 + row, M - 1) * K + chunk : W + (int64_t)(n0 + row - BM) * K + chunk;
+    // rows past M and N repeat the last one (their outputs are not stored)
+    const int n = n0 + row - BM;
+    src[i] = row < BM ? A + (int64_t)min(m0 + row, M - 1) * K + chunk
+                      : W + (int64_t)(kRagged ? min(n, N - 1) : n) * K + chunk;
   }
   const bool last = LAST == NT || tid < LAST;  // wave-uniform
   v4i stg[U][L];
@@ -1863,6 +1902,7 @@ __global__ __launch_bounds__(256 * KH, 1) void fp8_gemm_4n(
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
       const int n = n0 + i * 16 + 4 * g;
+      if (kRagged && n >= N) continue;
       const float4 sv = *(const float4*)(sb + n);
       const uint2 bb = bias ? *(const uint2*)(bias + n) : make_uint2(0u, 0u);
       const float sbe[4] = {sv.x, sv.y, sv.z, sv.w};
@@ -1886,11 +1926,11 @@ __global__ __launch_bounds__(256 * KH, 1) void fp8_gemm_4n(
   }
 }
 
-// One round of BM x 80 tiles (fp8_gemm_4n).
-template <bool kBf16, int kEpi, int BM, int U, int KH>
+// One round of BM x BN tiles (fp8_gemm_4n).
+template <bool kBf16, int kEpi, int BM, int BN, int U, int KH>
 hipError_t launch_narrow(const GemmArgs& g, hipStream_t st) {
-  const int tm = (g.M + BM - 1) / BM, tn = g.N / 80;
-  hipLaunchKernelGGL((fp8_gemm_4n<kBf16, kEpi, BM, U, KH>), dim3(tm * tn), dim3(256 * KH), 0, st, (const uint8_t*)g.A,
+  const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
+  hipLaunchKernelGGL((fp8_gemm_4n<kBf16, kEpi, BM, BN, U, KH>), dim3(tm * tn), dim3(256 * KH), 0, st, (const uint8_t*)g.A,
                      (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias, (uint16_t*)g.C, g.M, g.N,
                      g.K, g.ldc, tm, residual_args(g));
   return hipGetLastError();
@@ -1945,36 +1985,60 @@ SmallPlan small_plan(int M, int N, int K, bool allow_split) {
   return SmallPlan{2, splits_for(tiles(128, 128), 128)};
 }
 
-// Tile height of the narrow-tile plan (fp8_gemm_4n), or 0: one round of BM x 80 tiles where it
-// fills the CUs (N 5120: 64-row tiles at 129-256 rows, 128-row tiles at 449-512 rows with K below
-// 8192). Measured against the deep-K plans (W from HBM, graph-replayed, K 5120): M 200 20.2 ->
-// 15.8 us, M 256 21.9 -> 17.3 (no K split, no reduce launch), M 512 29.0 -> 24.6 (256 tiles
-// against 160), with the gated residual 31.8 -> 25.4. Where the deep-K plan splits K over
-// larger tiles it moves fewer bytes per CU and stays ahead: M 300 (3 x 64 tiles of 128 x 80)
-// 24.8 vs 22.3 us, M 512 x K 13824 56.3 vs 50.7.
-int narrow_bm(int M, int N, int K) {
-  if (N % 80 != 0 || K % 256 != 0 || M <= 128 || M > kSmallMaxM) return 0;
-  const int P = device_cus(), tn = N / 80;
-  const int t128 = ((M + 127) / 128) * tn, t64 = ((M + 63) / 64) * tn;
-  if (8 * t128 >= 7 * P && t128 <= P && K < 8192) return 128;
-  if (4 * t64 >= 3 * P && t64 <= P) return 64;
-  return 0;
+// Narrow-tile plan (fp8_gemm_4n): the shape with the fewest operand rows per tile (bm + bn) among
+// those whose tiles fill 3/4 of the CUs or more in one round, or {0, 0}. Below K 8192 only: with
+// longer K the deep-K plans split K over larger tiles, move fewer bytes per CU and stay ahead (M 200 x
+// N 4096 x K 16384 30.6 against 36.0 us, M 512 x N 5120 x K 13824 50.7 against 56.3). Only 48- and
+// 96-column tiles take a ragged N (5120 and 4096; the others' bounds checks cost them 2 %), and a last
+// column tile less than 2/3 full costs more than it gives; 16-column tiles are for a single row of
+// tiles (with more the rows outweigh them). Measured against the plans before (W from HBM): M 64 x N 4096 x
+// K 4096 10.6 -> 7.6 us, M 100 17.0 -> 8.2, M 200 17.3 -> 10.9, M 347 20.7 -> 15.5, M 512 22.1 -> 16.5;
+// M 64 x N 12288 15.9 -> 13.9, M 100 20.3 -> 17.3, x N 16384 26.9 -> 20.7; M 100 x N 5120 x K 5120
+// 16.5 -> 13.5, M 200 20.2 -> 15.8, M 347 24.2 -> 21.1, M 512 29.0 -> 24.6.
+TileShape narrow_plan(int M, int N, int K) {
+  TileShape best = {0, 0};
+  if (K % 256 != 0 || K >= 8192 || M <= 0 || M > kSmallMaxM) return best;
+  constexpr TileShape kShapes[] = {{64, 16}, {64, 32}, {64, 48}, {64, 64}, {64, 80}, {64, 96}, {128, 64}, {128, 80}};
+  const int64_t P = device_cus();
+  for (const TileShape& s : kShapes) {  // in the order of bm + bn
+    const int64_t tiles = (int64_t)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+    const int rest = N % s.bn;
+    if (rest != 0 && (!narrow_ragged(s.bn) || 3 * rest < 2 * s.bn)) continue;
+    if (tiles > P || 4 * tiles < 3 * P || (s.bn == 16 && M > 64)) continue;
+    best = s;
+    break;
+  }
+  return best;
+}
+
+// 129-512 rows whose one-tile workgroups fill 3/4 of the CUs in one round (launch_one_round)
+int64_t small_least_tiles() { return (3 * (int64_t)device_cus() + 3) / 4; }
+bool small_one_round(int M, int N, int K) {
+  return M > 128 && M <= kSmallMaxM && K % 128 == 0 && one_round_shape(M, N, small_least_tiles()).bm != 0;
 }
 
 template <bool kBf16, int kEpi>
 hipError_t launch_small_m(const GemmArgs& g, hipStream_t st) {
-  const int nbm = narrow_bm(g.M, g.N, g.K);
   // 128-row tiles with two waves per row group (each one of the two MFMA k-steps of a K step): 25.3 ->
-  // 24.6 us at M 512 x N 5120; 64-row tiles with one (two: 17.4 -> 18.3 us at M 256)
-  if (nbm == 128) return launch_narrow<kBf16, kEpi, 128, 2, 2>(g, st);
-  if (nbm == 64) return launch_narrow<kBf16, kEpi, 64, 2, 1>(g, st);
-  if (g.M > 256 && g.K % 128 == 0) {
-    // 257-512 rows where 256x128 tiles fill 3/4 of the CUs: one tile per workgroup with
-    // 128-byte K steps through the DMA ring (M 512 x N 15360: 43-45 us vs 47 for 128x256
-    // deep-K tiles, hipBLASLt 48; x N 13824 with GELU 42 vs 46). With fewer tiles (N 5120)
-    // the deep-K plans stay ahead (128x128 tiles: 30.3 vs 28.8 us).
-    const int tm = (g.M + 255) / 256, tn = (g.N + 127) / 128, P = device_cus();
-    if (4 * tm * tn >= 3 * P && tm * tn <= P) return launch_one_round_256x128<kBf16, kEpi>(g, tm, tn, st);
+  // 24.6 us at M 512 x N 5120; 64-row tiles with one (two: 17.4 -> 18.3 us at M 256, level elsewhere)
+  const TileShape np = narrow_plan(g.M, g.N, g.K);
+  if (np.bm == 128) {
+    if (np.bn == 64) return launch_narrow<kBf16, kEpi, 128, 64, 2, 2>(g, st);
+    return launch_narrow<kBf16, kEpi, 128, 80, 2, 2>(g, st);
+  }
+  if (np.bm == 64) {
+    if (np.bn == 16) return launch_narrow<kBf16, kEpi, 64, 16, 2, 1>(g, st);
+    if (np.bn == 32) return launch_narrow<kBf16, kEpi, 64, 32, 2, 1>(g, st);
+    if (np.bn == 48) return launch_narrow<kBf16, kEpi, 64, 48, 2, 1>(g, st);
+    if (np.bn == 64) return launch_narrow<kBf16, kEpi, 64, 64, 2, 1>(g, st);
+    if (np.bn == 80) return launch_narrow<kBf16, kEpi, 64, 80, 2, 1>(g, st);
+    return launch_narrow<kBf16, kEpi, 64, 96, 2, 1>(g, st);
+  }
+  if (small_one_round(g.M, g.N, g.K)) {
+    // one tile per workgroup through the DMA ring where its tiles fill 3/4 of the CUs (M 347 x N 12288
+    // x K 4096: 192x128 tiles 26.6 us, 256x128 28.5; x N 16384 28.9, 32.7; M 200 x N 16384: 128x128
+    // tiles 23.0 us, deep-K 25.2; M 512 x N 15360: 256x128 43-45 us, 128x256 deep-K 47, hipBLASLt 48)
+    return launch_one_round<kBf16, kEpi>(g, small_least_tiles(), st);
   }
   SmallPlan p = small_plan(g.M, g.N, g.K, true);
   if (p.splits > 1 && (g.workspace == nullptr || g.workspace_bytes < (int64_t)p.splits * g.M * g.N * 4))
@@ -2011,27 +2075,19 @@ hipError_t launch_gemm_t(const GemmArgs& g, hipStream_t st) {
                                      (uintptr_t)g.gate % 16 == 0));
   if (fast && g.M <= kSmallMaxM) return launch_small_m<kBf16, kEpi>(g, st);
   if (fast && g.M <= 2048 && g.K >= 4096 && g.K % 128 == 0) {
-    // Less than one round of 256x256 tiles: deep-K 128-row tiles. Measured with W
-    // from HBM, long K (the reference's 16384-wide FFN-down at 1024 / 1560 tokens):
-    // 1024 x 16384 x 4096: 79.3 us vs 89.3 (256x256 + split tail); 1560 x 16384 x 4096:
-    // 140.3 us vs 151.7. At K 4096 only where the 128-row tiles fit one round:
-    // 1024 x 4096 x 4096 26.9 us vs 30.1, 1560 x 4096 x 4096 42.6 vs 44.2, while
-    // 1024 x 4096 x 12288 (1.5 rounds of 128x256) takes 82.5 us vs 66.6.
-    // Where neither 128-row tile fits one round but 256x192 tiles do (1024 x 4096 x 12288:
-    // 256 tiles against 192 of 256x256), the 256x192 tiles fill every CU.
+    // Less than one round of 256x256 tiles: the smallest tile that fits one round. Where none of
+    // launch_one_round's does but 256x192 tiles do (1024 x 4096 x 12288: 256 tiles against 192 of
+    // 256x256), those fill every CU.
     const int P = device_cus();
     const int64_t t256 = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
-    const int64_t t128 = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
-    const int64_t t128x256 = (int64_t)((g.M + 127) / 128) * ((g.N + 255) / 256);
     const int64_t t256x192 = (int64_t)((g.M + 255) / 256) * ((g.N + 191) / 192);
-    const int64_t t256x128 = (int64_t)((g.M + 255) / 256) * ((g.N + 127) / 128);
     if (t256 < P) {
-      if (t128 <= P) return launch_deepk<kBf16, kEpi, 128, 128, 128, 3, 3>(g, 1, nullptr, st);
-      // 256x128 tiles with 128-byte steps where they fill more CUs than 128x256 (1560 rows: 224
-      // tiles against 208; 1560 x 4096 -> 4096 32.3 us vs 34.0, 1560 x 16384 -> 4096 109.7 vs 112.3)
-      if (t256x128 <= P && t256x128 > t128x256)
-        return launch_one_round_256x128<kBf16, kEpi>(g, (g.M + 255) / 256, (g.N + 127) / 128, st);
-      if (t128x256 <= P) return launch_deepk<kBf16, kEpi, 128, 256, 128, 2, 3>(g, 1, nullptr, st);
+      // long K with 128x128 tiles on less than 7/8 of the CUs: the deep-K kernel stays (600 x 13824 ->
+      // 5120, 200 tiles: 61.6 against 62.9 us)
+      const int64_t t128 = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+      if (g.K >= 8192 && 8 * t128 < 7 * P) return launch_deepk<kBf16, kEpi, 128, 128, 128, 3, 3>(g, 1, nullptr, st);
+      const hipError_t e = launch_one_round<kBf16, kEpi>(g, 0, st);
+      if (e != hipErrorNotFound) return e;
       if (t256x192 <= P) {
         // 256x192 tiles filling the CUs (1024 x 4096 -> 12288: 256 tiles): the persistent kernel,
         // one tile per workgroup (38.9 vs 43.9 us for the one-tile 32x32x64 kernel, bit-identical)
@@ -2143,7 +2199,7 @@ __global__ __launch_bounds__(256) void qkv_tail_norm_rope(const uint16_t* __rest
 }  // namespace
 
 int64_t fp8_gemm_workspace_bytes(int M, int N, int K) {
-  if (K < 64 || K % 64 != 0 || N % 8 != 0 || narrow_bm(M, N, K) != 0) return 0;
+  if (K < 64 || K % 64 != 0 || N % 8 != 0 || narrow_plan(M, N, K).bm != 0 || small_one_round(M, N, K)) return 0;
   const SmallPlan p = small_plan(M, N, K, true);
   return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
 }

@@ -490,3 +490,36 @@ def test_persistent_kernel_any_row_count(M, N, K, kind):
         ref = torch.addcmul(x, y, gate)
         got = jo.fp8_scaled_mm_gated_residual(a, w, sad, swd, x.to(DEV), gate.to(DEV), b)
         assert torch.equal(got.cpu(), ref)
+
+
+# one round of narrow tiles of every shape: 64 x 16, 32, 48 (ragged N), 64, 80, 96 (ragged N) and 128 x 64, 80, at the
+# first and last row counts of each, and one-tile workgroups of 128x128, 192x128, 256x128 and 128x256 (the last two
+# shapes: 513-2048 rows)
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 512), (64, 4096, 256), (65, 4096, 512), (100, 5120, 768), (16, 12288, 256),
+                                   (64, 16384, 512), (256, 4096, 768), (129, 5120, 512), (65, 12288, 256), (257, 4096, 512),
+                                   (320, 4096, 256), (128, 15360, 512), (347, 4096, 512), (384, 5120, 256),
+                                   (129, 12288, 384), (257, 12296, 384), (384, 16376, 256), (512, 12288, 128),
+                                   (600, 4104, 4096), (1021, 5120, 4096), (600, 12288, 4096)])
+@pytest.mark.parametrize("kind", ["plain", "residual"])
+def test_one_round_tile_shapes_exact(M, N, K, kind):
+    """Exact operands: every output bit is fixed; the row and column scales differ from row to row, so a row or a
+    column of another tile, or one past the end, shows."""
+    announce("gemm one round", M, N, K, kind)
+    import joyomni_ops as jo
+    rng = np.random.default_rng(M + N + K)
+    qa = f32_to_e4m3fn(rng.integers(-8, 9, (M, K)).astype(np.float32))
+    qw = f32_to_e4m3fn(rng.integers(-8, 9, (N, K)).astype(np.float32))
+    sa = (2.0 ** rng.integers(-12, -4, M)).astype(np.float32)
+    sw = (2.0 ** rng.integers(-12, -4, N)).astype(np.float32)
+    bias = f32_to_bf16((rng.integers(-64, 64, N) / 16).astype(np.float32))
+    exp_bits, _ = og.scaled_mm(qa, qw, sa, sw, bias)
+    if kind == "plain":
+        assert np.array_equal(u16(gemm(qa, qw, sa, sw, bias)), exp_bits)
+        return
+    g = gen(M)
+    x, gate = torch.randn(M, N, generator=g).bfloat16(), torch.randn(N, generator=g).bfloat16()
+    y = torch.from_numpy(exp_bits.view(np.int16)).view(torch.bfloat16)
+    b = torch.from_numpy(bias.view(np.int16)).view(torch.bfloat16).to(DEV)
+    got = jo.fp8_scaled_mm_gated_residual(to_dev_fp8(qa), to_dev_fp8(qw).t(), torch.from_numpy(sa).to(DEV),
+                                          torch.from_numpy(sw).to(DEV), x.to(DEV), gate.to(DEV), b)
+    assert torch.equal(got.cpu(), torch.addcmul(x, y, gate))
