@@ -233,8 +233,10 @@ JOY_API joy_status joy_fp8_qkv_norm_rope_cache(const void *mat_a, const void *ma
                                                int64_t cache_tokens, int cache_post_rope, void *scratch,
                                                int64_t scratch_bytes, void *stream);
 
-/* Bytes of scratch joy_fp8_qkv_norm_rope_cache needs with 16-byte aligned cos / sin and outputs of
- * token stride num_heads * head_dim (0 when every tile takes the fused epilogue). */
+/* Bytes of scratch joy_fp8_qkv_norm_rope_cache uses with 16-byte aligned cos / sin and outputs of
+ * token stride num_heads * head_dim (0 when every tile takes the fused epilogue). Shapes of less than
+ * a round of tiles use it to run the GEMM and the standalone kernel, which is faster there; those
+ * whose tiles could all take the fused epilogue accept less and then do. */
 JOY_API int64_t joy_fp8_qkv_norm_rope_cache_scratch_size(int64_t M, int64_t K, int64_t num_heads,
                                                          int64_t head_dim);
 

@@ -419,6 +419,7 @@ joy_status joy_fp8_qkv_norm_rope_cache(const void* mat_a, const void* mat_b, con
                 "fp8_qkv_norm_rope_cache: %lld bytes of scratch needed for this call, %lld given (cos/sin not "
                 "16-byte aligned or output offsets past 2^31 bytes need the M x 3*num_heads*head_dim bf16 buffer)",
                 (long long)need, (long long)scratch_bytes);
+  if (scratch_bytes < M * N * 2) g.C = nullptr;  // a smaller buffer, which this call can do without
   return hip_status(joy::launch_fp8_gemm_qkv(g, a, (int)head_dim, (hipStream_t)stream),
                     "fp8_qkv_norm_rope_cache launch");
 }

@@ -2217,8 +2217,12 @@ bool qkv_fusable(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
 }
 }  // namespace
 
-// Whether some tiles of the fused QKV projection go through the scratch: the persistent kernel's
-// epilogue takes the whole rounds, the tail kernel the sub-tiles of the last, partial one.
+// The fused epilogue pays from 7/8 of a round of 256x256 tiles on. With fewer the plain GEMM's smaller
+// tiles and the standalone norm/RoPE pass are faster (K 4096 -> 12288: 64 rows 28.5 -> 17.6 us, 300 rows
+// 37.0 -> 29.8, 600 rows 67.7 -> 42.6, 1024 rows (192 tiles) 59.3 -> 57.4; 1280 rows (240 tiles) fused
+// 62.5, else 66.6).
+static bool qkv_fills_round(const TilePlan& p) { return 8 * p.bulk >= 7 * device_cus(); }
+// Whether the fused form leaves tiles to the scratch: the sub-tiles of the last, partial round.
 static bool qkv_has_tail(int M, int N, int K) {
   const TilePlan p = tile_plan(M, N, K);
   return p.rem > 0 || p.sub_log2 == -4;
@@ -2236,7 +2240,8 @@ int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_
   a.num_heads = num_heads;
   a.n_tokens = a.table_len = M;
   a.q_out_stride = a.k_out_stride = a.kpre_stride = a.v_out_stride = a.v_out2_stride = (int64_t)num_heads * head_dim;
-  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(M, N, K)) return 0;
+  // without the fused form all rows go through it; a call with less runs the fused form if that needs none
+  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(M, N, K) && qkv_fills_round(tile_plan(M, N, K))) return 0;
   return (int64_t)M * N * 2;
 }
 
@@ -2248,7 +2253,9 @@ int64_t fp8_gemm_qkv_call_scratch_bytes(const GemmArgs& g, const NormRopeArgs& a
 
 hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int head_dim, hipStream_t st) {
   if (g.M == 0 || g.N == 0) return hipSuccess;
-  if (!qkv_fusable(g, a, head_dim) || (qkv_has_tail(g.M, g.N, g.K) && g.C == nullptr)) {
+  const TilePlan p = tile_plan(g.M, g.N, g.K);
+  const bool tail = qkv_has_tail(g.M, g.N, g.K);
+  if (!qkv_fusable(g, a, head_dim) || (g.C == nullptr ? tail : !qkv_fills_round(p))) {
     // the GEMM into C, then the standalone norm/RoPE kernel on it
     if (g.C == nullptr) return hipErrorInvalidValue;
     hipError_t e = launch_fp8_gemm(g, st);
@@ -2280,9 +2287,8 @@ hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int hea
   qe.heads = a.num_heads;
   qe.eps = a.eps;
   qe.kpre_rotated = a.cache_post_rope;
-  const TilePlan p = tile_plan(g.M, g.N, g.K);
-  const int P = device_cus();
-  if (p.bulk > 0) {
+  {
+    const int P = device_cus();
     hipLaunchKernelGGL((fp8_gemm_4q<true, kEpiQkv, 256>), dim3(p.bulk < P ? p.bulk : P), dim3(256), 0, st,
                        (const uint8_t*)g.A, (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias,
                        (uint16_t*)g.C, g.M, g.N, g.K, g.ldc, p.tiles_m, p.tiles_n, kGroupM, p.bulk, residual_args(g),
@@ -2290,7 +2296,7 @@ hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int hea
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (!qkv_has_tail(g.M, g.N, g.K)) return hipSuccess;
+  if (!tail) return hipSuccess;
   const uint16_t* c = (const uint16_t*)g.C;
   if (p.sub_log2 == 1) {
     hipLaunchKernelGGL((fp8_gemm_4h<true, kEpiPlain, 256, 128, 3>), dim3(p.rem << 1), dim3(256), 0, st,

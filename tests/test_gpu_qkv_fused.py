@@ -205,3 +205,30 @@ def test_no_ring_rows_written():
 def test_any_row_count(M):
     """Token counts that are no multiple of 4 take the fused epilogue like the others."""
     _run_both(M, 512, 4, 128, 90 + M, exact=True)
+
+
+@pytest.mark.parametrize("with_scratch", [True, False])
+def test_less_than_a_round_with_and_without_scratch(with_scratch):
+    """1024 rows x 32 heads (192 of 256 tiles) run as the GEMM and the standalone kernel where the scratch is
+    given, and in the fused epilogue where it is not: the same bits."""
+    announce("fp8 qkv norm rope less than a round", with_scratch)
+    import joyomni_ops as jo
+    from joyomni_ops import _lib
+    M, K, H, D = 1024, 512, 32, 128
+    E = H * D
+    a, b, sa, sw, bias, qw, kw, cos, sin = _problem(M, K, H, D, 77, True)
+    need = jo._LIB.joy_fp8_qkv_norm_rope_cache_scratch_size(M, K, H, D)
+    assert need == M * 3 * E * 2
+    ref = _outputs(M, H, D, 1, M, 78)
+    got = tuple(t.clone() for t in ref)
+    y = jo.fp8_scaled_mm(a, b, sa, sw, torch.bfloat16, bias)
+    jo.fused_qkv_norm_rope_cache(y, H, 1e-6, qw, kw, cos, sin, ref[0], ref[1], ref[3], ref[4], 0, 0, v_out=ref[2])
+    scratch = torch.empty(need if with_scratch else 16, dtype=torch.uint8, device=DEV)
+    _lib.check(jo._LIB, jo._LIB.joy_fp8_qkv_norm_rope_cache(
+        a.data_ptr(), b.data_ptr(), sa.data_ptr(), sw.data_ptr(), bias.data_ptr(), M, K, H, D, 1e-6, qw.data_ptr(),
+        kw.data_ptr(), cos.data_ptr(), sin.data_ptr(), got[0].data_ptr(), E, got[1].data_ptr(), E, got[2].data_ptr(), E,
+        got[3].data_ptr(), got[4].data_ptr(), 1, M, 0, 0, M, 0, scratch.data_ptr(), scratch.numel(),
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    for name, r, o in zip(("q_out", "k_out", "v_out", "ring K", "ring V"), ref, got):
+        assert torch.equal(u16_t(r), u16_t(o)), name
