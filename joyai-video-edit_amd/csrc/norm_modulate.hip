@@ -436,17 +436,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void n
   __shared__ __attribute__((aligned(16))) float sc1_l[N];
   __shared__ __attribute__((aligned(16))) float shf_l[N];
   const int t = threadIdx.x, lane = t & 63;
-  for (int i = t; i < N / 8; i += blockDim.x) {
-    float sc[8], sh[8];
-    unpack8<kFp16>(((const uint4*)a.scale)[i], sc);
-    unpack8<kFp16>(((const uint4*)a.shift)[i], sh);
+  // the modulation row's loads, then the first row's, then the modulation into LDS: with the first
+  // row loaded after the barrier, a wave that takes one row (up to 3072 rows) waited for memory twice
+  // (3072 x 4096: FP8 output 9.9 -> 9.3 us, bf16 11.9 -> 8.8; 10800 x 5120 32.8 -> 32.2, 41.7 -> 41.2)
+  constexpr int NS = (N / 8 + 255) / 256;
+  uint4 scv[NS], shv[NS];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      sc1_l[i * 8 + j] = 1.f + sc[j];
-      shf_l[i * 8 + j] = sh[j];
-    }
+  for (int k = 0; k < NS; ++k) {
+    const int i = min(t + 256 * k, N / 8 - 1);
+    scv[k] = ((const uint4*)a.scale)[i];
+    shv[k] = ((const uint4*)a.shift)[i];
   }
-  __syncthreads();
   const int waves = gridDim.x * (blockDim.x >> 6);
   int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (t >> 6);
   auto load_row = [&](int64_t r, uint4 (&v)[NV]) {
@@ -456,6 +456,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void n
   };
   uint4 nxt[NV];
   if (row < a.M) load_row(row, nxt);
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    const int i = t + 256 * k;
+    if (i >= N / 8) continue;
+    float sc[8], sh[8];
+    unpack8<kFp16>(scv[k], sc);
+    unpack8<kFp16>(shv[k], sh);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      sc1_l[i * 8 + j] = 1.f + sc[j];
+      shf_l[i * 8 + j] = sh[j];
+    }
+  }
+  __syncthreads();
   for (; row < a.M; row += waves) {
     // the row unpacked to fp32 once, then the next row's loads issued into the freed vectors
     float f[NV][8];
