@@ -523,3 +523,13 @@ def test_one_round_tile_shapes_exact(M, N, K, kind):
     got = jo.fp8_scaled_mm_gated_residual(to_dev_fp8(qa), to_dev_fp8(qw).t(), torch.from_numpy(sa).to(DEV),
                                           torch.from_numpy(sw).to(DEV), x.to(DEV), gate.to(DEV), b)
     assert torch.equal(got.cpu(), torch.addcmul(x, y, gate))
+
+
+# whole rounds of whole tile rows (256 and 512 tiles on 256 CUs) and 1, 60 and 128 rows below them; 129 rows take the
+# general plan
+@pytest.mark.parametrize("M,N,K", [(1025, 16384, 512), (1084, 16384, 512), (1152, 16384, 512), (1153, 16384, 512),
+                                   (2108, 16384, 512)])
+@pytest.mark.parametrize("kind", ["plain", "residual"])
+def test_rows_below_whole_rounds_exact(M, N, K, kind):
+    announce("gemm rows below whole rounds", M, N, K, kind)
+    test_one_round_tile_shapes_exact(M, N, K, kind)
