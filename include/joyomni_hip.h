@@ -209,8 +209,9 @@ JOY_API joy_status joy_fused_qkv_norm_rope_cache(const void *qkv, int64_t qkv_ro
  * reference counterpart): the image stream's QKV Fp8Linear (deploy/xvideo/models/dit/dit.py:409,
  * fp8_linear.py:114-141 on quantised activations) followed by the split, q/k RMSNorm, RoPE and
  * ring write of dit.py:409-451 -- joy_fp8_scaled_mm (bf16 out, [M, 3*num_heads*head_dim]) then
- * joy_fused_qkv_norm_rope_cache with seq_len = M and qkv its output, with the same results bit
- * for bit. Where the shape allows (head_dim 128, an even num_heads, K % 256 == 0, 32-bit
+ * joy_fused_qkv_norm_rope_cache with seq_len = M and qkv its output, with the same results (bit
+ * for bit wherever both GEMMs take the same tiles; a tile of another MFMA shape adds the products of
+ * a 128-byte K step in another order, which moves the last bf16 bit of a few outputs). Where the shape allows (head_dim 128, an even num_heads, K % 256 == 0, 32-bit
  * offsets) the GEMM's epilogue does the norm, rotation and writes itself, so the QKV rows never
  * reach HBM; the tiles of a last, partial round (and other shapes entirely) go through
  * `scratch` (bf16 [M, 3*num_heads*head_dim]) and the standalone kernel.
