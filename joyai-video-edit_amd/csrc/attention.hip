@@ -33,6 +33,7 @@
 // ds_read_b64_tr_b16 lane layout (measured on gfx950): within each group of 16
 // lanes, lane a points at 4 consecutive 16-bit values M[a][0..3] and lane i receives
 // M[4j + i/4][i % 4] for j = 0..3.
+#include <cfloat>
 #include <type_traits>
 
 #include "joy_common.hpp"
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_fwd_d128(AttnArgs a, int 
     const float mt = xor32_max(fmaxf(m, s[15]));
     const float m_cand = mt * sl2;
     // finite also where every score so far is -inf, so that such a tile adds nothing instead of NaN
-    st.m_new = fmaxf(fmaxf(m_run, m_cand), -3.0e38f);
+    st.m_new = fmaxf(fmaxf(m_run, m_cand), -FLT_MAX);
     st.alpha = __builtin_amdgcn_exp2f(m_run - st.m_new);
     st.rs = 0.f;
 #pragma unroll

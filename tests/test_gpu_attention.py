@@ -251,6 +251,20 @@ def test_key_split_with_parts_that_add_nothing():
     _check(out, q, k[keep], v[keep], "split -inf")
 
 
+@pytest.mark.parametrize("Lq,Lk,H", [(40, 100, 1), (64, 2048, 4)])  # unsplit; parts along the keys
+def test_scores_near_the_lowest_float(Lq, Lk, H):
+    """Finite scores close to the lowest float (masks written into the keys) are scores like others: the
+    highest of them take the whole weight, here every third key at -3.2e38 in units of log2 against -3.3e38."""
+    announce("attention lowest scores", Lq, Lk, H)
+    import joyomni_ops as jo
+    assert (jo._LIB.joy_attention_workspace_size(Lq, Lk, H) > 0) == (Lk == 2048)
+    q, k, v = _inputs(Lq, Lk, H, 21)
+    q.zero_()[:, :, 0] = 1
+    k[:, :, 0] = -3.3e38
+    k[1::3, :, 0] = -3.2e38
+    _check(_run(q, k, v, math.log(2)), q, k, v, "lowest scores", scale=math.log(2))
+
+
 def test_key_split_in_a_captured_graph():
     """sdpa_attention with a split captured into a HIP graph and replayed with eager work between."""
     announce("attention key split captured")
