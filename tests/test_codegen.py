@@ -94,3 +94,10 @@ def test_attention_occupancy_and_lds(kernels):
     (name, f), = [(k, v) for k, v in kernels["attention"].items() if "attn_fwd_d128" in k]
     assert f["vgpr_count"] <= 256, f"{name}: {f['vgpr_count']} VGPRs per lane, two waves per SIMD need <= 256"
     assert f["group_segment_fixed_size"] == 2 * 2 * 2 * 64 * 256, "K / V tiles: 2 buffers x 2 head slots x K, V"
+
+
+def test_attention_split_kernel_occupancy_and_lds(kernels):
+    """The kernel of calls with a key split: the same limits as the unsplit one."""
+    (name, f), = [(k, v) for k, v in kernels["attention"].items() if "attn_split_d128" in k]
+    assert f["vgpr_count"] <= 256 and f["private_segment_fixed_size"] == 0, name
+    assert f["group_segment_fixed_size"] == 2 * 2 * 2 * 64 * 256, "K / V tiles: 2 buffers x 2 head slots x K, V"
