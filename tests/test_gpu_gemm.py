@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import DEV, announce, gen, outlier_acts, u16, u8
+from gpu_util import DEV, announce, gen, kernels_of, outlier_acts, u16, u8
 from oracle import gemm as og
 from oracle import quant as oq
 from oracle.fp8 import bf16_to_f32, f32_to_bf16, f32_to_e4m3fn
@@ -430,11 +430,11 @@ def test_reference_tuned_shapes(M, K, N):
 @pytest.mark.parametrize("M,kind", [(4096, "plain"), (4100, "plain"), (4100, "gelu"), (4096, "nobias"),
                                     (4100, "fp16")])
 def test_persistent_rounds_match_per_tile_launch(M, kind):
-    """With K % 256 == 0 and M % 4 == 0 the 256x256 bulk runs as the persistent kernel; the same
-    rows computed in two calls of odd row counts (M % 4 != 0) take the one-tile-per-workgroup
-    kernel. Rows are independent and both sum each output's K products in the same order, so
-    the outputs must agree to the bit (M = 4100: a 4-row last tile row and a sub-tile tail
-    launch); sampled rows also hold the accumulation bound of the oracle."""
+    """Rows computed in one call and in two calls of odd row counts: other tiles, other last tile
+    rows (1 and 3 rows) and rows below whole rounds as a small GEMM. Rows are independent, and on
+    these operands every kernel's sums round alike, so the outputs agree to the bit; sampled rows
+    also hold the accumulation bound of the oracle. (Kernels against each other:
+    test_kernels_agree_on_random_operands.)"""
     N, K = 8192, 512
     announce("gemm persistent", M, N, K, kind)
     qa, sa, qw, sw, bias = quantized_problem(M, N, K, 4242 + M)
@@ -455,14 +455,13 @@ def test_persistent_rounds_match_per_tile_launch(M, kind):
                          f"persistent {kind}")
 
 
-# rows past the last whole tile row: 1, 3 (fewer than one 4-row group), 2 and 255, beside whole rounds (4099: 17 x 16
-# tiles, the last one with 3 rows) and a 256x192 plan (1021)
+# odd row counts in sub-tiles only (513, 1027, 2303: less than a quarter round), as whole rounds with 3 rows below them
+# (4099) and as persistent 256x192 tiles (1021); the persistent 256x256 tiles: test_persistent_kernel_last_tile_row
 @pytest.mark.parametrize("kind", ["plain", "gelu", "residual"])
 @pytest.mark.parametrize("M,N,K", [(513, 520, 512), (1027, 264, 768), (4099, 4096, 512), (2303, 1032, 512),
                                    (1021, 12288, 4096)])
 def test_persistent_kernel_any_row_count(M, N, K, kind):
-    """The persistent kernel with row counts that are no multiple of 4 and row scales that start 4 bytes past a
-    16-byte boundary: exact operands, so every row has its own scale and the output is fixed to the bit (GELU
+    """Row counts that are no multiple of 4 and row scales that start 4 bytes past a 16-byte boundary: exact operands, so every row has its own scale and the output is fixed to the bit (GELU
     against the oracle's own rounding of it, within one bf16 step)."""
     announce("gemm odd rows", M, N, K, kind)
     import joyomni_ops as jo
@@ -490,6 +489,35 @@ def test_persistent_kernel_any_row_count(M, N, K, kind):
         ref = torch.addcmul(x, y, gate)
         got = jo.fp8_scaled_mm_gated_residual(a, w, sad, swd, x.to(DEV), gate.to(DEV), b)
         assert torch.equal(got.cpu(), ref)
+
+
+# one partial round of persistent tiles (11 x 16 of 256x256, 4 x 64 of 256x192) whose last tile row has 1, 2, 3 rows
+# (fewer than one group of 4 row scales), 4, 5 and 255
+@pytest.mark.parametrize("kind", ["plain", "gelu", "residual"])
+@pytest.mark.parametrize("M,N,K,BN", [(2561, 4096, 512, 256), (2562, 4096, 512, 256), (2563, 4096, 512, 256),
+                                      (2565, 4096, 512, 256), (2815, 4096, 512, 256), (769, 12288, 4096, 192),
+                                      (770, 12288, 4096, 192)])
+def test_persistent_kernel_last_tile_row(M, N, K, BN, kind):
+    """The same exact construction at row counts whose every tile runs in the persistent kernel."""
+    _, names = kernels_of(lambda: test_persistent_kernel_any_row_count(M, N, K, kind))
+    epi = {"plain": 0, "gelu": 1, "residual": 2}[kind]
+    assert not names or [n for n in names if "gemm" in n] == [f"fp8_gemm_4q<true, {epi}, {BN}>"]
+
+
+def test_kernels_agree_on_random_operands():
+    """The persistent kernel (16x16x128 MFMAs) against the one-tile kernel (32x32x64) and the narrow tiles
+    (16x16x128) on the same random rows: all walk K in ascending 128-byte steps, and only the order inside a
+    step differs between the two MFMA shapes, so at most a few outputs differ, by a step of bf16 or two."""
+    M, N, K = 2048, 8192, 512
+    announce("gemm kernels against each other", M, N, K)
+    qa, sa, qw, sw, bias = quantized_problem(M, N, K, 99)
+    whole, names = kernels_of(lambda: u16(gemm(qa, qw, sa, sw, bias)))
+    assert not names or [n for n in names if "gemm" in n] == ["fp8_gemm_4q<true, 0, 256>"]
+    for rows, kernel in ((600, "fp8_gemm_4h<true, 0, 256, 128, 3>"), (128, "fp8_gemm_4n<true, 0, 64, 64, 2, 1>")):
+        part, names = kernels_of(lambda: u16(gemm(qa[:rows], qw, sa[:rows], sw, bias)))
+        assert not names or [n for n in names if "gemm" in n] == [kernel]
+        a, b = bf16_to_f32(part).astype(np.float64), bf16_to_f32(whole[:rows]).astype(np.float64)
+        assert (np.abs(a - b) <= 2.0 ** -6 * np.abs(b)).all() and np.count_nonzero(a != b) <= 1e-5 * a.size, kernel
 
 
 # one round of narrow tiles of every shape: 64 x 16, 32, 48 (ragged N), 64, 80, 96 (ragged N) and 128 x 64, 80, at the
