@@ -668,6 +668,9 @@ __device__ __forceinline__ void dma_buf16(uint32_t lds_addr, uint32_t voff, __am
                "s"(soff)
                : "m0");
 }
+__device__ __forceinline__ void dma_buf4(uint32_t lds_addr, uint32_t voff, __amdgpu_buffer_rsrc_t rsrc) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc) : "m0");
+}
 __device__ __forceinline__ void dma_glb16(uint32_t lds_addr, const void* p) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(p) : "m0");
 }
@@ -756,7 +759,9 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
   static_assert(kEpi == kEpiPlain || kEpi == kEpiGelu || kEpi == kEpiResidual || kEpi == kEpiQkv, "epilogues");
   static_assert(kEpi != kEpiQkv || (BN == 256 && kBf16), "fused QKV epilogue: 256-wide tiles (one head per wave), bf16");
   static_assert(BN == 128 || BN == 192 || BN == 256, "tile widths");
-  constexpr bool kCopyScales = kEpi == kEpiPlain || kEpi == kEpiGelu;
+  // how row scales reach side_lds for any row count (issue_side): 192-wide tiles have the registers for 4-byte DMAs
+  // (in 256-wide ones they cost 20-28 bytes of spills and 1-2 %)
+  constexpr bool kDwordScales = BN < 256, kCopyScales = !kDwordScales && (kEpi == kEpiPlain || kEpi == kEpiGelu);
   constexpr int BM = 256, KS = 128, NW = 4, S = 2;
   constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16, FH = FN / 2;
   constexpr int CPR = KS / 16, RPL = 64 / CPR;  // 8 chunks per row, 8 rows per DMA instruction
@@ -799,6 +804,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
       __builtin_amdgcn_make_buffer_rsrc(C, 0, (int)(((int64_t)(M - 1) * ldc + N) * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)((int64_t)M * K), 0x00020000);
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, (int)((int64_t)N * K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc((void*)sa, 0, M * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t rrs = __builtin_amdgcn_make_buffer_rsrc(
       (void*)res.ptr, 0, kEpi == kEpiResidual ? (int)(((int64_t)(M - 1) * res.ld + N) * 2) : 0, 0x00020000);
   const __amdgpu_buffer_rsrc_t grs =
@@ -834,11 +840,18 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
   };
   auto issue_side = [&](int mm, int nn) {
     const int lc = min(lane, (N - nn) / 4 - 1), lb = min(lane, (N - nn) / 8 - 1);
+    const void* pc = sb + nn + 4 * lc;
+    const void* pb = has_bias ? (const void*)(bias + nn + 8 * lb) : pc;
+    if constexpr (kDwordScales) {
+      // row scales, one a lane and 64 rows a wave (rows past M fall outside the descriptor's range and are never
+      // stored); waves 0 and 3 fill an unused kilobyte below
+      dma_buf4(lds_u32((lds_void*)(side_lds + wave * 256)), (uint32_t)(mm + wave * 64 + lane) * 4, srs);
+      dma_glb16(lds_u32((lds_void*)(side_lds + (wave == 0 ? 3 : wave) * 1024)), wave == 2 ? pb : pc);
+      return;
+    }
     // row scales, 4 a lane, none past M (M >= 4): whole groups only, and the last 4 of all rows to wave 3's
     // words (kCopyScales), or the last 4 in the last lane
     const void* ps = sa + (kCopyScales ? mm + 4 * min(lane, (M - mm) / 4 - 1) : min(mm + 4 * lane, M - 4));
-    const void* pc = sb + nn + 4 * lc;
-    const void* pb = has_bias ? (const void*)(bias + nn + 8 * lb) : pc;
     const void* src = wave == 0 ? ps : (wave == 2 ? pb : (kCopyScales && wave == 3 ? (const void*)(sa + M - 4) : pc));
     dma_glb16(lds_u32((lds_void*)(side_lds + wave * 1024)), src);
   };
@@ -953,7 +966,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
       const uint16_t* bias_l = (const uint16_t*)(side_lds + 2048);
       uint8_t* stage = stage_lds + wave * STAGE;
       const int mw = tm0 + wm * WTM, nw0 = tn0 + wn * WTN;
-      // In the last tile row the last M % 4 row scales are not in their place (issue_side). Plain and
+      // In the last tile row of 256-wide tiles the last M % 4 row scales are not in their place (issue_side). Plain and
       // GELU epilogues copy them there from wave 3's words, which hold the last 4: every wave
       // writes the same values, before its own reads of them, and the other lanes copy an unused word
       // onto itself (a branch costs the K loop 52 bytes of spills). The others, whose registers that
@@ -965,7 +978,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
         side[mine ? (M & 252) + lane_e : 832 + lane_e] = side[mine ? 772 - odd + lane_e : 832 + lane_e];
         asm volatile("" ::: "memory");
       }
-      auto row_scale = [&](int r) { return sa_l[kCopyScales ? r : r + max(0, (r & ~3) - (M - 4 - tm0))]; };
+      auto row_scale = [&](int r) { return sa_l[kCopyScales || kDwordScales ? r : r + max(0, (r & ~3) - (M - 4 - tm0))]; };
       typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
       if constexpr (kEpi == kEpiQkv) {
         // this wave's 128 columns are one head of q, k or v (the three blocks are 256-aligned)
