@@ -1606,28 +1606,44 @@ int quarter_tiles(const TilePlan& p, int N) { return p.rem * 4 + (N + 127) / 128
 
 template <bool kBf16, int kEpi>
 hipError_t launch_small_m(const GemmArgs& g, hipStream_t st);
+TileShape narrow_plan(int M, int N, int K);
+
+// Whole tile rows that fill whole rounds, and at most 128 rows below them: those run as a small GEMM of their own,
+// whose tiles move half the operand bytes of the quarter tiles that the plan would cut the padded last tile row
+// into. 3120 x 4096 -> 16384 with GELU (12 x 64 tiles and 48 rows) 185 -> 173 us, 3172 rows 188 -> 181, 1100 rows
+// 83.0 -> 74.4, 2050 x 4096 -> 8192 77.4 -> 58.1. With 65 to 128 rows only where narrow tiles take them: unsplit
+// 128-row tiles on 8 to 32 CUs last longer than the quarter tiles (4164 x 8192 -> 4096 116.5 against 121.3 us, 4224 x
+// 16384 -> 4096 223.5 against 233, 8260 x 4096 -> 2048 65.3 against 68.2; up to 64 rows 64-row tiles do not: 4160 x
+// 8192 -> 4096 116.3 against 109.0, 8256 x 4096 -> 2048 65.2 against 61.9).
+int rest_rows(const GemmArgs& g) {
+  const int last = g.M % 256;
+  if (last == 0 || last > 128 || g.M <= 256 || !persistent_ok(g)) return 0;
+  if (((g.M / 256) * ((g.N + 255) / 256)) % device_cus() != 0) return 0;
+  return last <= 64 || narrow_plan(last, g.N, g.K).bm != 0 ? last : 0;
+}
+// The GEMM of the last `rows` rows, without a workspace.
+GemmArgs last_rows(const GemmArgs& g, int rows) {
+  GemmArgs r = g;
+  const int64_t m = g.M - rows;
+  r.M = rows;
+  r.A = (const uint8_t*)g.A + m * g.K;
+  r.scales_a = g.scales_a + m;
+  r.C = (uint16_t*)g.C + m * g.ldc;
+  if (g.residual) r.residual = (const uint16_t*)g.residual + m * g.ldr;
+  r.workspace = nullptr;
+  r.workspace_bytes = 0;
+  return r;
+}
 
 // The tile plan's launches, on the same stream.
 template <bool kBf16, int kEpi>
 hipError_t launch_4w(const GemmArgs& g, hipStream_t st) {
   const int P = device_cus();
-  // Whole tile rows that fill whole rounds, and at most 128 rows below them: those as a small GEMM of
-  // their own, whose narrow tiles move half the operand bytes of the quarter tiles that the plan would
-  // cut the padded last tile row into. 3120 x 4096 -> 16384 with GELU (12 x 64 tiles and 48 rows) 185 ->
-  // 173 us, 3172 rows 188 -> 181, 1100 rows 83.0 -> 74.4, 2050 x 4096 -> 8192 77.4 -> 58.1.
-  const int last = g.M % 256;
-  if (last > 0 && last <= 128 && g.M > 256 && persistent_ok(g) && ((g.M / 256) * ((g.N + 255) / 256)) % P == 0) {
-    GemmArgs head = g, rest = g;
-    const int64_t m = head.M = g.M - last;
-    rest.M = last;
-    rest.A = (const uint8_t*)g.A + m * g.K;
-    rest.scales_a = g.scales_a + m;
-    rest.C = (uint16_t*)g.C + m * g.ldc;
-    if (g.residual) rest.residual = (const uint16_t*)g.residual + m * g.ldr;
-    rest.workspace = nullptr;
-    rest.workspace_bytes = 0;
+  if (const int rest = rest_rows(g)) {
+    GemmArgs head = g;
+    head.M = g.M - rest;
     const hipError_t e = launch_4w<kBf16, kEpi>(head, st);
-    return e != hipSuccess ? e : launch_small_m<kBf16, kEpi>(rest, st);
+    return e != hipSuccess ? e : launch_small_m<kBf16, kEpi>(last_rows(g, rest), st);
   }
   const TilePlan tp = tile_plan(g.M, g.N, g.K);
   const int tiles_m = tp.tiles_m, tiles_n = tp.tiles_n, bulk = tp.bulk, rem = tp.rem, sub_log2 = tp.sub_log2;

@@ -561,3 +561,13 @@ def test_one_round_tile_shapes_exact(M, N, K, kind):
 def test_rows_below_whole_rounds_exact(M, N, K, kind):
     announce("gemm rows below whole rounds", M, N, K, kind)
     test_one_round_tile_shapes_exact(M, N, K, kind)
+
+
+# 60 rows: 64-row tiles; 68 rows where no narrow tiles fill the CUs: the tile plan's quarter tiles; 128 rows where some do
+@pytest.mark.parametrize("M,N,kernel", [(8252, 2048, "fp8_gemm_4k"), (8260, 2048, "fp8_gemm_4h<true, 0, 128, 128, 4>"),
+                                        (1152, 16384, "fp8_gemm_4n")])
+def test_rows_below_whole_rounds_route(M, N, kernel):
+    announce("gemm rows below whole rounds, route", M, N)
+    _, names = kernels_of(lambda: test_one_round_tile_shapes_exact(M, N, 512, "plain"))
+    gemms = [n for n in names if "gemm" in n]
+    assert not names or (gemms[0] == "fp8_gemm_4q<true, 0, 256>" and gemms[1].startswith(kernel) and len(gemms) == 2)
