@@ -209,12 +209,15 @@ JOY_API joy_status joy_fused_qkv_norm_rope_cache(const void *qkv, int64_t qkv_ro
  * reference counterpart): the image stream's QKV Fp8Linear (deploy/xvideo/models/dit/dit.py:409,
  * fp8_linear.py:114-141 on quantised activations) followed by the split, q/k RMSNorm, RoPE and
  * ring write of dit.py:409-451 -- joy_fp8_scaled_mm (bf16 out, [M, 3*num_heads*head_dim]) then
- * joy_fused_qkv_norm_rope_cache with seq_len = M and qkv its output, with the same results (bit
- * for bit wherever both GEMMs take the same tiles; a tile of another MFMA shape adds the products of
- * a 128-byte K step in another order, which moves the last bf16 bit of a few outputs). Where the shape allows (head_dim 128, an even num_heads, K % 256 == 0, 32-bit
+ * joy_fused_qkv_norm_rope_cache with seq_len = M and qkv its output, with the same results bit
+ * for bit (operands 16-byte aligned, and the scratch that the size query gives): every row runs in the
+ * GEMM kernel that joy_fp8_scaled_mm gives it. Exception: shapes of 7/8 to one round of 256 x 256 tiles
+ * with M <= 512 or K >= 8192, whose GEMM alone takes kernels that add the products of a 128-byte K step in
+ * another order (the last bf16 bit of a few outputs in ten million).
+ * Where the shape allows (head_dim 128, an even num_heads, K % 256 == 0, 32-bit
  * offsets) the GEMM's epilogue does the norm, rotation and writes itself, so the QKV rows never
- * reach HBM; the tiles of a last, partial round (and other shapes entirely) go through
- * `scratch` (bf16 [M, 3*num_heads*head_dim]) and the standalone kernel.
+ * reach HBM; the tiles of a last, partial round, a few rows below whole rounds (and other shapes entirely)
+ * go through `scratch` (bf16 [M, 3*num_heads*head_dim]) and the standalone kernel.
  * GEMM arguments as joy_fp8_scaled_mm (mat_b: [3*num_heads*head_dim, K] e4m3fn, bias bf16 or
  * NULL); norm/RoPE/ring arguments as joy_fused_qkv_norm_rope_cache (cos/sin [M, head_dim/2]).
  * scratch: 16-byte aligned device memory of at least joy_fp8_qkv_norm_rope_cache_scratch_size
@@ -236,8 +239,9 @@ JOY_API joy_status joy_fp8_qkv_norm_rope_cache(const void *mat_a, const void *ma
 
 /* Bytes of scratch joy_fp8_qkv_norm_rope_cache uses with 16-byte aligned cos / sin and outputs of
  * token stride num_heads * head_dim (0 when every tile takes the fused epilogue). Shapes of less than
- * a round of tiles use it to run the GEMM and the standalone kernel, which is faster there; those
- * whose tiles could all take the fused epilogue accept less and then do. */
+ * 7/8 of a round of tiles use it to run the GEMM and the standalone kernel, which is faster there, and with
+ * it the GEMM's workspace, after the rows; they accept M * 3 * num_heads * head_dim * 2 bytes (a GEMM without
+ * a K split) and, where all tiles could take the fused epilogue, less (they then do). */
 JOY_API int64_t joy_fp8_qkv_norm_rope_cache_scratch_size(int64_t M, int64_t K, int64_t num_heads,
                                                          int64_t head_dim);
 

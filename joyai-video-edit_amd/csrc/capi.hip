@@ -420,6 +420,11 @@ joy_status joy_fp8_qkv_norm_rope_cache(const void* mat_a, const void* mat_b, con
                 "16-byte aligned or output offsets past 2^31 bytes need the M x 3*num_heads*head_dim bf16 buffer)",
                 (long long)need, (long long)scratch_bytes);
   if (scratch_bytes < M * N * 2) g.C = nullptr;  // a smaller buffer, which this call can do without
+  const int64_t ws_offset = joy::qkv_workspace_offset(M, N);
+  if (scratch_bytes > ws_offset) {  // the split-K workspace of the unfused form's GEMM
+    g.workspace = (char*)scratch + ws_offset;
+    g.workspace_bytes = scratch_bytes - ws_offset;
+  }
   return hip_status(joy::launch_fp8_gemm_qkv(g, a, (int)head_dim, (hipStream_t)stream),
                     "fp8_qkv_norm_rope_cache launch");
 }

@@ -1529,7 +1529,7 @@ bool persistent_ok(const GemmArgs& g) {
 // -> 4096 21.4 -> 19.4, 800 x 16384 -> 4096 67.7 -> 62.3 (1024 rows: level); 192x128 tiles where 128x128
 // take more than a round: 800 x 5120 -> 5120 33.3 -> 27.8, 1024 x 5120 -> 5120 41.7 -> 30.2; 128x256:
 // 600 x 4096 -> 12288 37.7 -> 33.9. The 3-slot ring of 256x128 tiles also beats the persistent
-// 16x16x128 kernel here (1560 x 4096 -> 4096: 29.0 vs 30.0 us; bit-identical).
+// 16x16x128 kernel here (1560 x 4096 -> 4096: 29.0 vs 30.0 us; the same bits on the timed inputs).
 template <bool kBf16, int kEpi, int BM, int BN, int S>
 hipError_t launch_4h(const GemmArgs& g, hipStream_t st) {
   const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
@@ -1562,8 +1562,10 @@ hipError_t launch_one_round(const GemmArgs& g, int64_t least_tiles, hipStream_t 
 // the rest of the last, partial round split into 4 (128x128, sub_log2 2) or 2 (256x128, sub_log2 1)
 // sub-tiles so that more CUs share that round (not split where it is nearly full), or, with a short
 // last tile row, sub_log2 -4 (decode_job). The plain, GELU and residual GEMMs and the fused QKV
-// projection share it; the result does not depend on the split (every output element sums its K
-// products in the same order).
+// projection share it. Every output element adds its K products in ascending 128-byte steps whatever the split;
+// within a step the sub-tiles' 32x32x64 MFMAs add in another order than the persistent kernel's 16x16x128, which on
+// random operands moves the last bf16 bit of a few outputs in ten million. So a row's last bits can depend on
+// the row count of the call; two calls of the same shape give the same bits.
 struct TilePlan {
   int tiles_m, tiles_n, bulk, rem, sub_log2;
 };
@@ -2140,7 +2142,7 @@ hipError_t launch_gemm_t(const GemmArgs& g, hipStream_t st) {
       if (e != hipErrorNotFound) return e;
       if (t256x192 <= P) {
         // 256x192 tiles filling the CUs (1024 x 4096 -> 12288: 256 tiles): the persistent kernel,
-        // one tile per workgroup (38.9 vs 43.9 us for the one-tile 32x32x64 kernel, bit-identical)
+        // one tile per workgroup (38.9 vs 43.9 us for the one-tile 32x32x64 kernel, the same bits on the timed inputs)
         const int tm = (g.M + 255) / 256, tn = (g.N + 191) / 192;
         if (persistent_ok(g)) {
           hipLaunchKernelGGL((fp8_gemm_4q<kBf16, kEpi, 192>), dim3(tm * tn), dim3(256), 0, st, (const uint8_t*)g.A,
@@ -2248,6 +2250,9 @@ __global__ __launch_bounds__(256) void qkv_tail_norm_rope(const uint16_t* __rest
 
 }  // namespace
 
+// Where the GEMM's workspace begins in the scratch of a QKV projection: after the [M, N] bf16 rows.
+int64_t qkv_workspace_offset(int64_t M, int64_t N) { return (M * N * 2 + 255) / 256 * 256; }
+
 int64_t fp8_gemm_workspace_bytes(int M, int N, int K) {
   if (K < 64 || K % 64 != 0 || N % 8 != 0 || narrow_plan(M, N, K).bm != 0 || small_one_round(M, N, K)) return 0;
   const SmallPlan p = small_plan(M, N, K, true);
@@ -2272,10 +2277,13 @@ bool qkv_fusable(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
 // 37.0 -> 29.8, 600 rows 67.7 -> 42.6, 1024 rows (192 tiles) 59.3 -> 57.4; 1280 rows (240 tiles) fused
 // 62.5, else 66.6).
 static bool qkv_fills_round(const TilePlan& p) { return 8 * p.bulk >= 7 * device_cus(); }
-// Whether the fused form leaves tiles to the scratch: the sub-tiles of the last, partial round.
-static bool qkv_has_tail(int M, int N, int K) {
-  const TilePlan p = tile_plan(M, N, K);
-  return p.rem > 0 || p.sub_log2 == -4;
+// The plan of a fused QKV projection: the tile plan of the rows above rest_rows, so that every row runs in the kernel
+// that the plain GEMM gives it and the op's results are the two-op sequence's.
+static TilePlan qkv_plan(const GemmArgs& g) { return tile_plan(g.M - rest_rows(g), g.N, g.K); }
+// Whether the fused form leaves tiles to the scratch: the sub-tiles of the last, partial round, or rows below whole rounds.
+static bool qkv_has_tail(const GemmArgs& g) {
+  const TilePlan p = qkv_plan(g);
+  return rest_rows(g) > 0 || p.rem > 0 || p.sub_log2 == -4;
 }
 
 int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_dim) {
@@ -2290,35 +2298,54 @@ int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_
   a.num_heads = num_heads;
   a.n_tokens = a.table_len = M;
   a.q_out_stride = a.k_out_stride = a.kpre_stride = a.v_out_stride = a.v_out2_stride = (int64_t)num_heads * head_dim;
-  // without the fused form all rows go through it; a call with less runs the fused form if that needs none
-  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(M, N, K) && qkv_fills_round(tile_plan(M, N, K))) return 0;
-  return (int64_t)M * N * 2;
+  if (qkv_fusable(g, a, head_dim) && qkv_fills_round(qkv_plan(g))) return qkv_has_tail(g) ? (int64_t)M * N * 2 : 0;
+  // without the fused form all rows go through it, and the GEMM's workspace follows them; a call with less runs the
+  // fused form if that needs none, or the GEMM without a split
+  return qkv_workspace_offset(M, N) + fp8_gemm_workspace_bytes(M, N, K);
 }
 
 int64_t fp8_gemm_qkv_call_scratch_bytes(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
   if (g.M <= 0 || g.N <= 0) return 0;
-  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(g.M, g.N, g.K)) return 0;
+  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(g)) return 0;
   return (int64_t)g.M * g.N * 2;
+}
+
+// The standalone norm/RoPE/ring pass over the rows of g.C from row0 on.
+static hipError_t norm_rope_rows(const GemmArgs& g, const NormRopeArgs& a, int head_dim, int64_t row0, hipStream_t st) {
+  NormRopeArgs b = a;
+  const uint16_t* c = (const uint16_t*)g.C + row0 * g.ldc;
+  const int64_t eh = (int64_t)a.num_heads * head_dim;
+  b.q_in = a.q_out ? c : nullptr;
+  b.k_in = c + eh;
+  b.v_in = (a.v_out || a.v_out2) ? c + 2 * eh : nullptr;
+  b.in_stride = g.ldc;
+  if (row0 > 0) {
+    if (b.q_out) b.q_out += row0 * b.q_out_stride;
+    if (b.k_out) b.k_out += row0 * b.k_out_stride;
+    if (b.v_out2) b.v_out2 += row0 * b.v_out2_stride;
+    b.cache_tokens = max((int64_t)0, a.cache_tokens - row0);
+    b.kpre_out = b.kpre_out && b.cache_tokens > 0 ? b.kpre_out + row0 * b.kpre_stride : nullptr;
+    b.v_out = b.v_out && b.cache_tokens > 0 ? b.v_out + row0 * b.v_out_stride : nullptr;
+    if (!b.v_out && !b.v_out2) b.v_in = nullptr;
+    b.cos += row0 * (head_dim / 2);
+    b.sin += row0 * (head_dim / 2);
+    b.n_tokens -= row0;
+    b.table_len -= row0;
+  }
+  return launch_qk_norm_rope(b, head_dim, st);
 }
 
 hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int head_dim, hipStream_t st) {
   if (g.M == 0 || g.N == 0) return hipSuccess;
-  const TilePlan p = tile_plan(g.M, g.N, g.K);
-  const bool tail = qkv_has_tail(g.M, g.N, g.K);
+  const TilePlan p = qkv_plan(g);
+  const bool tail = qkv_has_tail(g);
   if (!qkv_fusable(g, a, head_dim) || (g.C == nullptr ? tail : !qkv_fills_round(p))) {
     // the GEMM into C, then the standalone norm/RoPE kernel on it
     if (g.C == nullptr) return hipErrorInvalidValue;
-    hipError_t e = launch_fp8_gemm(g, st);
-    if (e != hipSuccess) return e;
-    NormRopeArgs b = a;
-    const uint16_t* c = (const uint16_t*)g.C;
-    const int64_t eh = (int64_t)a.num_heads * head_dim;
-    b.q_in = a.q_out ? c : nullptr;
-    b.k_in = c + eh;
-    b.v_in = (a.v_out || a.v_out2) ? c + 2 * eh : nullptr;
-    b.in_stride = g.ldc;
-    return launch_qk_norm_rope(b, head_dim, st);
+    const hipError_t e = launch_fp8_gemm(g, st);
+    return e != hipSuccess ? e : norm_rope_rows(g, a, head_dim, 0, st);
   }
+  const int rest = rest_rows(g), head_rows = g.M - rest;
   QkvEpi qe{};
   uint16_t* dst[5] = {a.q_out, a.k_out, a.kpre_out, a.v_out, a.v_out2};
   const int64_t stride[5] = {a.q_out_stride, a.k_out_stride, a.kpre_stride, a.v_out_stride, a.v_out2_stride};
@@ -2341,12 +2368,16 @@ hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int hea
     const int P = device_cus();
     hipLaunchKernelGGL((fp8_gemm_4q<true, kEpiQkv, 256>), dim3(p.bulk < P ? p.bulk : P), dim3(256), 0, st,
                        (const uint8_t*)g.A, (const uint8_t*)g.W, g.scales_a, g.scales_b, (const uint16_t*)g.bias,
-                       (uint16_t*)g.C, g.M, g.N, g.K, g.ldc, p.tiles_m, p.tiles_n, kGroupM, p.bulk, residual_args(g),
-                       qe);
+                       (uint16_t*)g.C, head_rows, g.N, g.K, g.ldc, p.tiles_m, p.tiles_n, kGroupM, p.bulk,
+                       residual_args(g), qe);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (!tail) return hipSuccess;
+  if (rest > 0) {  // whole rounds above them: no sub-tiles
+    const hipError_t e = launch_fp8_gemm(last_rows(g, rest), st);
+    return e != hipSuccess ? e : norm_rope_rows(g, a, head_dim, head_rows, st);
+  }
   const uint16_t* c = (const uint16_t*)g.C;
   if (p.sub_log2 == 1) {
     hipLaunchKernelGGL((fp8_gemm_4h<true, kEpiPlain, 256, 128, 3>), dim3(p.rem << 1), dim3(256), 0, st,

@@ -128,6 +128,8 @@ int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_
 // The scratch a given call needs: also counts what only the call's pointers and strides decide
 // (16-byte aligned cos / sin, 31-bit output offsets), which send it to the unfused path.
 int64_t fp8_gemm_qkv_call_scratch_bytes(const GemmArgs& g, const NormRopeArgs& a, int head_dim);
+// Where the workspace of the unfused form's GEMM begins in that scratch, after the [M, N] bf16 rows.
+int64_t qkv_workspace_offset(int64_t M, int64_t N);
 // Workspace bytes the GEMM of this shape can use on the current device (0: none).
 int64_t fp8_gemm_workspace_bytes(int M, int N, int K);
 hipError_t launch_norm_modulate(const NormModArgs& a, hipStream_t st);

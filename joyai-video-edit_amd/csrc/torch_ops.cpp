@@ -13,6 +13,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 #include <tuple>
@@ -338,8 +339,8 @@ void fp8_qkv_norm_rope_cache(const Tensor& mat_a, const Tensor& mat_b, const Ten
   // outputs whose byte offsets pass 2^31 take the unfused path, through an [M, N] bf16 buffer
   const std::pair<const OptTensor&, int64_t> outs[] = {{q_out, r.q_stride}, {k_out, r.k_stride}, {v_out, r.v_stride}};
   for (const auto& [t, stride] : outs)
-    if (t && (s.M * stride + H * D) * 2 > 0x7fffffffLL) bytes = s.M * s.N * 2;
-  // the tiles that do not take the fused epilogue pass through this [M, N] bf16 buffer
+    if (t && (s.M * stride + H * D) * 2 > 0x7fffffffLL) bytes = std::max(bytes, s.M * s.N * 2);
+  // the tiles that do not take the fused epilogue pass through this [M, N] bf16 buffer (and the workspace after it)
   const Tensor scratch = bytes > 0 ? bytes_like(bytes, mat_a) : Tensor();
   check_status(joy_fp8_qkv_norm_rope_cache(
       ptr(mat_a), ptr(mat_b), (const float*)ptr(scales_a), (const float*)ptr(scales_b), ptr(bias), s.M, s.K, H, D,

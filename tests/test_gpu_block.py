@@ -469,12 +469,26 @@ def test_block_torch_sdpa_backend_matches_hip_attention():
 
 @pytest.mark.parametrize("E,H,write_only", [(512, 4, False), (1024, 8, False), (1024, 8, True)])
 def test_block_fused_qkv_matches_unfused(E, H, write_only):
-    """The video stream's QKV projection with its q/k norm, RoPE and ring write in the GEMM
+    """The video stream's QKV projection with its q/k norm, RoPE and ring write in one op
     (fuse_qkv=True, the default) and as the GEMM followed by fused_qkv_norm_rope_cache: the same
-    block outputs and ring contents bit for bit (also the cache-only forward)."""
+    block outputs and ring contents bit for bit (also the cache-only forward). At these sizes the op runs
+    the two kernels itself; in the GEMM's epilogue: test_block_fused_qkv_epilogue_matches_unfused."""
+    _block_fused_against_unfused(E, H, write_only, 12, 20)
+
+
+@pytest.mark.parametrize("hh,ww,write_only", [(44, 25, False), (30, 52, False), (30, 52, True)])
+def test_block_fused_qkv_epilogue_matches_unfused(hh, ww, write_only):
+    """The same at sizes whose projection runs in the fused epilogue: 1100 tokens (240 tiles) and 1560 (a whole
+    round and quarter tiles) of a 4096-wide block."""
+    from gpu_util import kernels_of
+    _, names = kernels_of(lambda: _block_fused_against_unfused(4096, 32, write_only, hh, ww, FFN=1024))
+    assert not names or "fp8_gemm_4q<true, 4, 256>" in names
+
+
+def _block_fused_against_unfused(E, H, write_only, hh, ww, FFN=None):
     from joyomni_ops.dit_block import CachedChunk, KVRing, QuantizedDoubleStreamBlock
-    announce("block fused qkv vs unfused", E, H, write_only)
-    FFN, T, hh, ww = 3 * E, 32, 12, 20
+    announce("block fused qkv vs unfused", E, H, write_only, hh, ww)
+    FFN, T = FFN or 3 * E, 32
     L, D = hh * ww, E // H
     img = torch.randn(1, L, E, generator=gen(727)).to(torch.bfloat16).to(DEV)
     txt = torch.randn(1, T, E, generator=gen(728)).to(torch.bfloat16).to(DEV)

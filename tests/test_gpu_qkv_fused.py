@@ -4,18 +4,19 @@
 on every output: rotated Q and K, the ring slot's K (normalised or rotated) and V, the second V
 destination, and the ring rows and slots it must not touch.
 
-Cases cover the three ways a tile reaches the outputs: the persistent kernel's fused epilogue,
-the sub-tiles of a last partial round (stored plainly, then the tail kernel), and the fallback of
-shapes the fused epilogue does not take (odd head counts, head_dim 64, K % 256 != 0), which runs
-the two-op sequence itself. Where the plain GEMM's kernel choice for a shape may differ from the
-fused op's tile plan, operands are exact small integers with power-of-two scales, so every GEMM
-output is exact whatever the summation order and the comparison isolates the norm/RoPE/ring work.
+Cases cover the ways a row reaches the outputs: the persistent kernel's fused epilogue (from 7/8 of a
+round of 256x256 tiles on), the sub-tiles of a last partial round (stored plainly, then the tail
+kernel), the rows below whole rounds (a small GEMM, then the standalone kernel), and the two-op
+sequence itself with fewer tiles and for shapes the epilogue does not take (odd head counts, head_dim
+64, K % 256 != 0). Most operands are exact small integers with power-of-two scales, so every GEMM
+output is exact whatever the summation order and the comparison isolates the norm/RoPE/ring work;
+test_same_gemm_kernels_as_the_two_ops takes operands whose sums show the order.
 """
 import numpy as np
 import pytest
 import torch
 
-from gpu_util import DEV, announce, gen, u16
+from gpu_util import DEV, announce, gen, kernels_of, u16
 from oracle import rope as orope
 from oracle.fp8 import f32_to_bf16, f32_to_e4m3fn
 
@@ -35,7 +36,15 @@ def _problem(M, K, H, D, seed, exact):
     tables [M, D/2]."""
     rng = np.random.default_rng(seed)
     N = 3 * H * D
-    if exact:
+    if exact == "order":
+        # positive products over 30 binary places in the first half of K, taken back but for a few per cent of them
+        # in the second: the sums pass through 100 times their result, whose bf16 bits then show the order of adding
+        x, y = (np.exp(1.5 * rng.standard_normal((r, K // 2))).clip(2.0 ** -8, 400).astype(np.float32) for r in (M, N))
+        z = np.where(rng.random(y.shape) < 0.05, np.roll(y, 1, axis=1), y)
+        a, w = _fp8(np.concatenate([x, -x], axis=1)), _fp8(np.concatenate([y, z], axis=1))
+        sa = torch.from_numpy((2.0 ** rng.integers(-10, -5, M)).astype(np.float32)).to(DEV)
+        sw = torch.from_numpy((2.0 ** rng.integers(-8, -4, N)).astype(np.float32)).to(DEV)
+    elif exact:
         a = _fp8(rng.integers(-8, 9, (M, K)).astype(np.float32))
         w = _fp8(rng.integers(-8, 9, (N, K)).astype(np.float32))
         sa = torch.from_numpy((2.0 ** rng.integers(-10, -5, M)).astype(np.float32)).to(DEV)
@@ -111,12 +120,12 @@ def u16_t(t):
 
 @pytest.mark.parametrize("M,K,H,D", [
     (4352, 1024, 32, 128),  # whole rounds through the fused epilogue + q, k and v tiles as quarter sub-tiles
-    (2048, 1024, 8, 128),   # less than one round: every tile through the sub-tile launch
-    (1000, 2048, 16, 128),  # ragged M
-    (777, 512, 5, 128),     # odd head count: fallback
-    (300, 1024, 6, 64),     # head_dim 64: fallback
-    (640, 640, 4, 128),     # K % 256 != 0: fallback
-    (1002, 1024, 8, 128),   # M % 4 != 0
+    (2048, 1024, 8, 128),   # 96 tiles, less than 7/8 of a round: the two ops themselves
+    (1000, 2048, 16, 128),  # the same, ragged M
+    (777, 512, 5, 128),     # odd head count: the two ops
+    (300, 1024, 6, 64),     # head_dim 64: the two ops
+    (640, 640, 4, 128),     # K % 256 != 0: the two ops
+    (1002, 1024, 8, 128),   # less than 7/8 of a round, M % 4 != 0
 ])
 def test_exact_equals_gemm_then_norm_rope(M, K, H, D):
     announce("fp8 qkv norm rope exact", M, K, H, D)
@@ -139,8 +148,8 @@ def test_cache_only_forward():
 
 def test_block_shape_random_operands():
     """The block's video stream at the benchmark's size (10800 tokens, 40 x 128 heads, K 5120) on
-    random quantised operands: the fused op and the two-op sequence run the same GEMM kernels, so
-    every output is bit-identical (the whole rounds through the fused epilogue, the last round's
+    random quantised operands: the fused op and the two-op sequence give every row the same GEMM kernel,
+    so every output is bit-identical (the whole rounds through the fused epilogue, the last round's
     V tiles as quarter sub-tiles)."""
     announce("fp8 qkv norm rope block shape", 10800, 5120, 40, 128)
     _run_both(10800, 5120, 40, 128, 13, exact=False)
@@ -203,8 +212,62 @@ def test_no_ring_rows_written():
 
 @pytest.mark.parametrize("M", [515, 4353, 4354])  # a partial last tile row of 3, 1 and 2 rows
 def test_any_row_count(M):
-    """Token counts that are no multiple of 4 take the fused epilogue like the others."""
+    """Token counts that are no multiple of 4 and less than 7/8 of a round of tiles: the two ops
+    (whole rounds: test_fused_epilogue_row_counts)."""
     _run_both(M, 512, 4, 128, 90 + M, exact=True)
+
+
+Q4, H128, H256 = "fp8_gemm_4q<true, 4, 256>", "fp8_gemm_4h<true, 0, 128, 128, 4>", "fp8_gemm_4h<true, 0, 256, 128, 3>"
+
+
+def _fused_op_kernels(names):
+    """The kernels after the two-op sequence's norm/RoPE kernel: the fused op's."""
+    i = next((i for i, n in enumerate(names) if n.startswith("qk_norm_rope_kernel")), -1)
+    return names[i + 1:]
+
+
+@pytest.mark.parametrize("M,kernels", [
+    (2305, [Q4]), (2306, [Q4]), (2307, [Q4]),  # 10 x 48 tiles: 1, 2 and 3 rows in the last tile row
+    (2816, [Q4, H128, "qkv_tail_norm_rope<128>"]), (4353, [Q4, H256, "qkv_tail_norm_rope<256>"]),
+    (4355, [Q4, H256, "qkv_tail_norm_rope<256>"]),
+    # a short last tile row as quarter tiles beside the leftover ones
+    (1560, [Q4, H128, "qkv_tail_norm_rope<128>"]), (1563, [Q4, H128, "qkv_tail_norm_rope<128>"]),
+])
+@pytest.mark.parametrize("cache_tokens", [-1, 1500])
+def test_fused_epilogue_row_counts(M, kernels, cache_tokens):
+    """Row counts, odd ones among them, through the fused epilogue and every form of its tail; the ring takes all
+    rows or the first 1500."""
+    announce("fp8 qkv norm rope row counts", M, cache_tokens)
+    _, names = kernels_of(lambda: _run_both(M, 512, 32, 128, M, exact=True, cache_tokens=cache_tokens))
+    assert not names or _fused_op_kernels(names) == kernels
+
+
+# rows below whole rounds, sub-tiles of both kinds, and split-K GEMMs of few tiles (with their workspace)
+@pytest.mark.parametrize("M,K,H,fused", [(4100, 1024, 32, True), (4223, 1024, 32, True), (3120, 1024, 32, True),
+                                         (1560, 1024, 32, True), (64, 4096, 4, False), (200, 8192, 4, False)])
+def test_same_gemm_kernels_as_the_two_ops(M, K, H, fused):
+    """Operands whose rounded sums show the order in which a kernel adds them: the op gives every row the GEMM
+    kernel that fp8_scaled_mm gives it, so the results are still the two ops' bit for bit."""
+    import joyomni_ops as jo
+    announce("fp8 qkv norm rope same kernels", M, K, H)
+    _, names = kernels_of(lambda: _run_both(M, K, H, 128, M + K, exact="order"))
+    assert not names or (Q4 in _fused_op_kernels(names)) == fused
+    if M == 4100:  # the operands do show it: 32x32x64 against 16x16x128 MFMAs
+        a, b, sa, sw, bias = _problem(M, K, H, 128, M + K, "order")[:5]
+        whole = jo.fp8_scaled_mm(a, b, sa, sw, torch.bfloat16, bias)[:600]
+        part = jo.fp8_scaled_mm(a[:600], b, sa[:600], sw, torch.bfloat16, bias)
+        torch.cuda.synchronize()
+        assert 0 < int((whole != part).sum()) < 0.2 * whole.numel()
+
+
+@pytest.mark.parametrize("outputs", ["ring", "no ring", "q"])
+def test_rows_below_whole_rounds_with_fewer_outputs(outputs):
+    """4100 tokens: the 4 rows below whole rounds with the ring alone (all of it above them), without ring rows, and
+    with Q alone beside the ring."""
+    announce("fp8 qkv norm rope rows below whole rounds", outputs)
+    kw = {"ring": dict(with_q=False, with_k=False, with_v=False, cache_tokens=4096),
+          "no ring": dict(cache_tokens=0), "q": dict(with_k=False, with_v=False, cache_tokens=4098, pre_rope=False)}
+    _run_both(4100, 512, 32, 128, 31, exact=True, **kw[outputs])
 
 
 @pytest.mark.parametrize("with_scratch", [True, False])
