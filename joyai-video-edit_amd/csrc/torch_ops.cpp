@@ -633,8 +633,11 @@ void fused_norm_scale_shift_fp8(const Tensor& x, const OptTensor& gamma, const O
 
 }  // namespace
 
+// The C ABI that these operators were compiled for: compared by the package when it has loaded the library (an
+// exception during the load itself would end the process).
+extern "C" __attribute__((visibility("default"))) int joy_torch_abi_version(void) { return JOY_ABI_VERSION; }
+
 TORCH_LIBRARY_IMPL(joyomni_ops, CUDA, m) {
-  TORCH_CHECK(joy_abi_version() == JOY_ABI_VERSION, "libjoyomni_hip.so and libjoyomni_torch.so were built apart");
   m.impl("sgl_per_token_quant_fp8", sgl_per_token_quant_fp8);
   m.impl("per_token_quant_fp8", per_token_quant_fp8);
   m.impl("fp8_scaled_mm", fp8_scaled_mm);

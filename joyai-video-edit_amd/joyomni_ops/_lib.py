@@ -112,10 +112,16 @@ def load_ops() -> None:
     if not os.path.exists(TORCH_LIB_PATH):
         raise ImportError(f"{os.path.basename(TORCH_LIB_PATH)} not found beside {LIB_NAME}; build it first "
                           "(make -C joyai-video-edit_amd/csrc)")
+    name = os.path.basename(TORCH_LIB_PATH)
     try:
         torch.ops.load_library(TORCH_LIB_PATH)
+        version = ctypes.CDLL(TORCH_LIB_PATH).joy_torch_abi_version()
     except OSError as e:
         raise ImportError(str(e)) from e
+    except AttributeError as e:
+        raise ImportError(f"{name} was built for another ABI version than {ABI_VERSION}") from e
+    if version != ABI_VERSION:
+        raise ImportError(f"{name} was built for ABI version {version}, not {ABI_VERSION}")
 
 
 def check(lib: ctypes.CDLL, status: int) -> None:

@@ -102,3 +102,18 @@ def test_visual_rope_tables_match_oracle():
     assert torch.equal(c0, c1) and torch.equal(s0, s1)
     with pytest.raises(ValueError, match="temporal ids"):
         rope.visual_rope_tables((2, 4, 6), 3, temporal_ids=torch.tensor([0, 1]))
+
+
+@pytest.mark.parametrize("source", ["int joy_torch_abi_version(void) { return 0; }", "int unrelated(void) { return 0; }"])
+def test_operator_library_of_another_build_is_an_import_error(source, tmp_path, monkeypatch):
+    """libjoyomni_torch.so from another ABI version: an ImportError, not the end of the process."""
+    import shutil
+    import subprocess
+    from joyomni_ops import _lib
+    if shutil.which("gcc") is None:
+        pytest.skip("gcc not available")
+    path = tmp_path / "libjoyomni_torch.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(path), "-x", "c", "-"], input=source.encode(), check=True)
+    monkeypatch.setattr(_lib, "TORCH_LIB_PATH", str(path))
+    with pytest.raises(ImportError, match="ABI version"):
+        _lib.load_ops()
