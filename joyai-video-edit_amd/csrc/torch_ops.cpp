@@ -8,9 +8,12 @@
 // call through a Python implementation (dispatch, checks, ctypes) took 11 us for the quantiser, 18 for
 // the GEMM, 21 for attention and 35 for the fused QKV projection, longer than their kernels; here 4.4,
 // 7.0, 5.3 and 11.5 us (Fp8Linear on 64 rows 38.1 -> 17.9 us a call).
+#include <Python.h>
+
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/library.h>
 
 #include <algorithm>
@@ -54,7 +57,21 @@ void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t
 void* ptr(const Tensor& t) { return t.data_ptr(); }
 void* ptr(const OptTensor& t) { return t ? t->data_ptr() : nullptr; }
 
-void check_status(joy_status st) { TORCH_CHECK(st == JOY_OK, joy_last_error()); }
+// A C-ABI refusal is the package's JoyError (a RuntimeError; the argument checks here raise RuntimeError
+// itself). The caller may have released the GIL.
+void check_status(joy_status st) {
+  if (st == JOY_OK) return;
+  const PyGILState_STATE gil = PyGILState_Ensure();
+  PyObject* module = PyImport_ImportModule("joyomni_ops._lib");
+  PyObject* type = module ? PyObject_GetAttrString(module, "JoyError") : nullptr;
+  PyErr_SetString(type ? type : PyExc_RuntimeError, joy_last_error());
+  Py_XDECREF(type);
+  Py_XDECREF(module);
+  python_error error;
+  error.persist();
+  PyGILState_Release(gil);
+  throw error;
+}
 
 int dtype_code(ScalarType t) { return t == at::kBFloat16 ? JOY_DTYPE_BF16 : t == at::kHalf ? JOY_DTYPE_FP16 : JOY_DTYPE_FP32; }
 

@@ -283,3 +283,21 @@ def test_key_split_in_a_captured_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("through", ["wrapper", "torch.ops"])
+def test_c_abi_refusals_are_joy_errors(through):
+    """What the C ABI refuses under an operator is raised as the package's JoyError, with its text; an operator's own
+    argument check as a RuntimeError that is none."""
+    announce("JoyError", through)
+    import joyomni_ops as jo
+    from joyomni_ops import _lib
+    op = jo.sdpa_attention if through == "wrapper" else torch.ops.joyomni_ops.sdpa_attention
+    x = torch.zeros(1, 4, 2, 64, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(_lib.JoyError, match="head_dim=128 only"):
+        op(x, x, x)
+    with pytest.raises(RuntimeError, match="same shape") as e:
+        op(x, x, x[:, :2])
+    assert not isinstance(e.value, _lib.JoyError)
+    y = torch.zeros(1, 4, 2, 128, dtype=torch.bfloat16, device=DEV)
+    assert not op(y, y, y).any()  # and the next call is an ordinary one
