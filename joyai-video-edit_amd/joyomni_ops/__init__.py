@@ -123,24 +123,24 @@ _ops = torch.ops.joyomni_ops
 _lib.load_ops()
 
 
-def _check(cond: bool, msg: str) -> None:
-    if not cond:
-        raise RuntimeError(msg)
+_DEVICE = torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA)
 
 
 def _quant_impl(input, output_q, output_s, rounding):
-    """The quantiser by its C-ABI rounding, for device tensors (others are refused by name)."""
-    for name, t in (("input", input), ("output_q", output_q), ("output_s", output_s)):
-        _check(t.is_cuda, f"{name} must be a CUDA tensor")
-    _ops.per_token_quant_fp8(input, output_q, output_s, rounding == _lib.JOY_QUANT_DIVIDE)
+    """The quantiser's device implementation by C-ABI rounding code, called for tensors of any device
+    (its own checks refuse the others)."""
+    if rounding not in (_lib.JOY_QUANT_DIVIDE, _lib.JOY_QUANT_RECIPROCAL):
+        raise _lib.JoyError("rounding must be JOY_QUANT_DIVIDE or JOY_QUANT_RECIPROCAL")
+    _ops.per_token_quant_fp8.default.redispatch(_DEVICE, input, output_q, output_s,
+                                                rounding == _lib.JOY_QUANT_DIVIDE)
 
 
 def _scaled_mm_impl(mat_a, mat_b, scales_a, scales_b, out_dtype, bias, epilogue):
-    """The GEMM by its C-ABI epilogue, for device tensors (others are refused by name)."""
-    _check(mat_a.is_cuda, "mat_a must be a CUDA tensor")
-    _check(mat_b.is_cuda, "mat_b must be a CUDA tensor")
-    op = _ops.fp8_scaled_mm_gelu_tanh if epilogue == _lib.JOY_EPILOGUE_GELU_TANH else _ops.fp8_scaled_mm
-    return op(mat_a, mat_b, scales_a, scales_b, out_dtype, bias)
+    """The GEMM's device implementation by C-ABI epilogue code, likewise."""
+    op = {_lib.JOY_EPILOGUE_NONE: _ops.fp8_scaled_mm, _lib.JOY_EPILOGUE_GELU_TANH: _ops.fp8_scaled_mm_gelu_tanh}.get(epilogue)
+    if op is None:
+        raise _lib.JoyError(f"unknown epilogue {epilogue}")
+    return op.default.redispatch(_DEVICE, mat_a, mat_b, scales_a, scales_b, out_dtype, bias)
 
 
 # --------------------------------------------------------------------------

@@ -58,6 +58,15 @@ def test_cpu_tensors_rejected_like_reference():
         jo._scaled_mm_impl(a, a.t(), s, s, torch.bfloat16, None, 0)
 
 
+def test_unknown_codes_refused():
+    x = torch.zeros(4, 32, dtype=torch.bfloat16)
+    q, s = torch.empty(4, 32, dtype=torch.float8_e4m3fn), torch.empty(4, 1)
+    with pytest.raises(jo._lib.JoyError, match="rounding must be"):
+        jo._quant_impl(x, q, s, 2)
+    with pytest.raises(jo._lib.JoyError, match="unknown epilogue 2"):
+        jo._scaled_mm_impl(q, q.t(), s, s, torch.bfloat16, None, 2)
+
+
 def test_fp8_linear_api_surface():
     assert fp8_linear.available()
     assert fp8_linear.backend() == "joyomni_ops/gfx950-hip"
