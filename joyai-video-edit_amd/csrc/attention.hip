@@ -121,8 +121,8 @@ __device__ __forceinline__ float xor32_sum(float v) {
 // and sum in the workspace, and attn_combine adds a group's parts in key order. A workgroup takes
 // one part only: a loop over several in one workgroup costs 114 VGPR spills. What the kernel is
 // bound by stays as above (LDS operand reads and power); the split fills idle CUs. Measured against
-// the unsplit call: 512 x 8000 x 32 heads 179 -> 80 us, 859 x 5000 x 32 131 -> 98 us, 5000 x 5000 x 40
-// 571 -> 496 us, 3467 x 11267 x 32 636 -> 629 us. (wave is moved to a scalar register, so that the DMA's
+// the unsplit call, the second launch included: 512 x 8000 x 32 heads 183 -> 73 us, 859 x 5000 x 32 132 -> 95,
+// 5000 x 5000 x 40 554 -> 472, 3467 x 11267 x 32 626 -> 603. (wave is moved to a scalar register, so that the DMA's
 // LDS addresses are scalars: 250 -> 248 VGPRs with the split's code, 0.5-3 % faster unsplit.)
 constexpr int kWaves = 8;
 constexpr int kPartBlock = 64 * 64 + 64;        // floats per query block of a part: O, then m and l of 32 queries

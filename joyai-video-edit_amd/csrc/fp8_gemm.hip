@@ -1797,9 +1797,10 @@ hipError_t launch_deepk(const GemmArgs& g, int splits, float* ws, hipStream_t st
 // ---------------------------------------------------------------------------
 // Narrow tiles for small M (16-512 tokens: the condition stream, small chunks): BM x BN tiles, BM = 64
 // or 128, so that one round of tiles fills the CUs without a K split (narrow_plan). These GEMMs are
-// bound by the operand bytes each CU streams, (BM + BN) x K per tile, at 40-80 GB/s per CU when the
-// operands come partly from HBM: a copy of the one-tile DMA kernel without its MFMAs and LDS reads
-// takes 27.6 of 28.9 us at M 347 x N 16384 x K 4096, and three or four steps in flight instead of two,
+// bound by the operand bytes each CU streams, (BM + BN) x K per tile, at 40-50 GB/s per CU with W
+// from HBM (65-71 with W in the memory-side cache): a copy of the one-tile DMA kernel without its MFMAs and LDS reads
+// takes 27.3 of 27.7 us at M 347 x N 12288 x K 4096 and 29.5 of 31.4 at N 16384 (MFMAs busy 0.33 and 0.43 of the
+// time, 0.05 to 0.24 in the narrow tiles), and three or four steps in flight instead of two,
 // or K orders that differ from panel to panel, change nothing. So the shape that fills one round
 // with the fewest BM + BN is the fastest.
 //
@@ -2174,7 +2175,7 @@ hipError_t launch_gemm_t(const GemmArgs& g, hipStream_t st) {
 // (20 to 40 MB), so it wants loads in flight: a workgroup that walked a whole sub-tile, 16 rows at
 // a time, left 160 to 256 workgroups with one load each in flight: the whole op at 1560 x 4096 ->
 // 12288 109.5 -> 91.0 us (with the tile plan's quarter tiles for its 24-row last tile row), at
-// 3120 rows 163.9 -> 154.6, at 300 rows 49.3 -> 37.0, at 10800 x 5120 -> 15360 710 -> 695.
+// 3120 rows 163.9 -> 154.6, at 10800 x 5120 -> 15360 710 -> 695.
 constexpr int kTailRows = 32;
 template <int BMs>
 __global__ __launch_bounds__(256) void qkv_tail_norm_rope(const uint16_t* __restrict__ C, int64_t ldc, int M,
