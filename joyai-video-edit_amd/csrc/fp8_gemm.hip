@@ -759,9 +759,10 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
   static_assert(kEpi == kEpiPlain || kEpi == kEpiGelu || kEpi == kEpiResidual || kEpi == kEpiQkv, "epilogues");
   static_assert(kEpi != kEpiQkv || (BN == 256 && kBf16), "fused QKV epilogue: 256-wide tiles (one head per wave), bf16");
   static_assert(BN == 128 || BN == 192 || BN == 256, "tile widths");
-  // how row scales reach side_lds for any row count (issue_side): 192-wide tiles have the registers for 4-byte DMAs
-  // (in 256-wide ones they cost 20-28 bytes of spills and 1-2 %)
-  constexpr bool kDwordScales = BN < 256, kCopyScales = !kDwordScales && (kEpi == kEpiPlain || kEpi == kEpiGelu);
+  // how row scales reach side_lds for any row count (issue_side): copied into place in plain and GELU epilogues, by
+  // 4-byte DMAs in 192-wide gated-residual ones (in 256-wide tiles those cost 20-28 bytes of spills and 1-2 %), else
+  // looked up
+  constexpr bool kCopyScales = kEpi == kEpiPlain || kEpi == kEpiGelu, kDwordScales = kEpi == kEpiResidual && BN < 256;
   constexpr int BM = 256, KS = 128, NW = 4, S = 2;
   constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16, FH = FN / 2;
   constexpr int CPR = KS / 16, RPL = 64 / CPR;  // 8 chunks per row, 8 rows per DMA instruction
@@ -840,6 +841,9 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
   };
   auto issue_side = [&](int mm, int nn) {
     const int lc = min(lane, (N - nn) / 4 - 1), lb = min(lane, (N - nn) / 8 - 1);
+    // row scales, 4 a lane, none past M (M >= 4): whole groups only, and the last 4 of all rows to wave 3's
+    // words (kCopyScales), or the last 4 in the last lane
+    const void* ps = sa + (kCopyScales ? mm + 4 * min(lane, (M - mm) / 4 - 1) : min(mm + 4 * lane, M - 4));
     const void* pc = sb + nn + 4 * lc;
     const void* pb = has_bias ? (const void*)(bias + nn + 8 * lb) : pc;
     if constexpr (kDwordScales) {
@@ -849,9 +853,6 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
       dma_glb16(lds_u32((lds_void*)(side_lds + (wave == 0 ? 3 : wave) * 1024)), wave == 2 ? pb : pc);
       return;
     }
-    // row scales, 4 a lane, none past M (M >= 4): whole groups only, and the last 4 of all rows to wave 3's
-    // words (kCopyScales), or the last 4 in the last lane
-    const void* ps = sa + (kCopyScales ? mm + 4 * min(lane, (M - mm) / 4 - 1) : min(mm + 4 * lane, M - 4));
     const void* src = wave == 0 ? ps : (wave == 2 ? pb : (kCopyScales && wave == 3 ? (const void*)(sa + M - 4) : pc));
     dma_glb16(lds_u32((lds_void*)(side_lds + wave * 1024)), src);
   };
@@ -966,7 +967,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_4q(
       const uint16_t* bias_l = (const uint16_t*)(side_lds + 2048);
       uint8_t* stage = stage_lds + wave * STAGE;
       const int mw = tm0 + wm * WTM, nw0 = tn0 + wn * WTN;
-      // In the last tile row of 256-wide tiles the last M % 4 row scales are not in their place (issue_side). Plain and
+      // In the last tile row the last M % 4 row scales are not in their place (issue_side). Plain and
       // GELU epilogues copy them there from wave 3's words, which hold the last 4: every wave
       // writes the same values, before its own reads of them, and the other lanes copy an unused word
       // onto itself (a branch costs the K loop 52 bytes of spills). The others, whose registers that
