@@ -240,8 +240,8 @@ JOY_API joy_status joy_fp8_qkv_norm_rope_cache(const void *mat_a, const void *ma
 /* Bytes of scratch joy_fp8_qkv_norm_rope_cache uses with 16-byte aligned cos / sin and outputs of
  * token stride num_heads * head_dim (0 when every tile takes the fused epilogue). Shapes of less than
  * 7/8 of a round of tiles use it to run the GEMM and the standalone kernel, which is faster there, and with
- * it the GEMM's workspace, after the rows; they accept M * 3 * num_heads * head_dim * 2 bytes (a GEMM without
- * a K split) and, where all tiles could take the fused epilogue, less (they then do). */
+ * it the GEMM's workspace, after the rows; M * 3 * num_heads * head_dim * 2 bytes do as well (a GEMM without
+ * a K split). Shapes whose tiles could all take the fused epilogue accept less, and then do. */
 JOY_API int64_t joy_fp8_qkv_norm_rope_cache_scratch_size(int64_t M, int64_t K, int64_t num_heads,
                                                          int64_t head_dim);
 

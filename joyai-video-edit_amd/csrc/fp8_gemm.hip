@@ -2279,14 +2279,10 @@ bool qkv_fusable(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
 // 37.0 -> 29.8, 600 rows 67.7 -> 42.6, 1024 rows (192 tiles) 59.3 -> 57.4; 1280 rows (240 tiles) fused
 // 62.5, else 66.6).
 static bool qkv_fills_round(const TilePlan& p) { return 8 * p.bulk >= 7 * device_cus(); }
-// The plan of a fused QKV projection: the tile plan of the rows above rest_rows, so that every row runs in the kernel
-// that the plain GEMM gives it and the op's results are the two-op sequence's.
-static TilePlan qkv_plan(const GemmArgs& g) { return tile_plan(g.M - rest_rows(g), g.N, g.K); }
-// Whether the fused form leaves tiles to the scratch: the sub-tiles of the last, partial round, or rows below whole rounds.
-static bool qkv_has_tail(const GemmArgs& g) {
-  const TilePlan p = qkv_plan(g);
-  return rest_rows(g) > 0 || p.rem > 0 || p.sub_log2 == -4;
-}
+// The plan of a fused QKV projection is the tile plan of the rows above rest_rows, so that every row runs in the
+// kernel that the plain GEMM gives it and the op's results are the two-op sequence's (without scratch, of all rows).
+// Whether a plan leaves tiles to the scratch: the sub-tiles of the last, partial round.
+static bool has_tail(const TilePlan& p) { return p.rem > 0 || p.sub_log2 == -4; }
 
 int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_dim) {
   if (M <= 0 || N <= 0) return 0;
@@ -2300,7 +2296,9 @@ int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_
   a.num_heads = num_heads;
   a.n_tokens = a.table_len = M;
   a.q_out_stride = a.k_out_stride = a.kpre_stride = a.v_out_stride = a.v_out2_stride = (int64_t)num_heads * head_dim;
-  if (qkv_fusable(g, a, head_dim) && qkv_fills_round(qkv_plan(g))) return qkv_has_tail(g) ? (int64_t)M * N * 2 : 0;
+  const int rest = rest_rows(g);
+  const TilePlan p = tile_plan(M - rest, N, K);
+  if (qkv_fusable(g, a, head_dim) && qkv_fills_round(p)) return rest > 0 || has_tail(p) ? (int64_t)M * N * 2 : 0;
   // without the fused form all rows go through it, and the GEMM's workspace follows them; a call with less runs the
   // fused form if that needs none, or the GEMM without a split
   return qkv_workspace_offset(M, N) + fp8_gemm_workspace_bytes(M, N, K);
@@ -2308,7 +2306,7 @@ int64_t fp8_gemm_qkv_scratch_bytes(int M, int N, int K, int num_heads, int head_
 
 int64_t fp8_gemm_qkv_call_scratch_bytes(const GemmArgs& g, const NormRopeArgs& a, int head_dim) {
   if (g.M <= 0 || g.N <= 0) return 0;
-  if (qkv_fusable(g, a, head_dim) && !qkv_has_tail(g)) return 0;
+  if (qkv_fusable(g, a, head_dim) && !has_tail(tile_plan(g.M, g.N, g.K))) return 0;
   return (int64_t)g.M * g.N * 2;
 }
 
@@ -2339,15 +2337,14 @@ static hipError_t norm_rope_rows(const GemmArgs& g, const NormRopeArgs& a, int h
 
 hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int head_dim, hipStream_t st) {
   if (g.M == 0 || g.N == 0) return hipSuccess;
-  const TilePlan p = qkv_plan(g);
-  const bool tail = qkv_has_tail(g);
-  if (!qkv_fusable(g, a, head_dim) || (g.C == nullptr ? tail : !qkv_fills_round(p))) {
+  const int rest = g.C == nullptr ? 0 : rest_rows(g), head_rows = g.M - rest;
+  const TilePlan p = tile_plan(head_rows, g.N, g.K);
+  if (!qkv_fusable(g, a, head_dim) || (g.C == nullptr ? has_tail(p) : !qkv_fills_round(p))) {
     // the GEMM into C, then the standalone norm/RoPE kernel on it
     if (g.C == nullptr) return hipErrorInvalidValue;
     const hipError_t e = launch_fp8_gemm(g, st);
     return e != hipSuccess ? e : norm_rope_rows(g, a, head_dim, 0, st);
   }
-  const int rest = rest_rows(g), head_rows = g.M - rest;
   QkvEpi qe{};
   uint16_t* dst[5] = {a.q_out, a.k_out, a.kpre_out, a.v_out, a.v_out2};
   const int64_t stride[5] = {a.q_out_stride, a.k_out_stride, a.kpre_stride, a.v_out_stride, a.v_out2_stride};
@@ -2375,11 +2372,11 @@ hipError_t launch_fp8_gemm_qkv(const GemmArgs& g, const NormRopeArgs& a, int hea
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (!tail) return hipSuccess;
   if (rest > 0) {  // whole rounds above them: no sub-tiles
     const hipError_t e = launch_fp8_gemm(last_rows(g, rest), st);
     return e != hipSuccess ? e : norm_rope_rows(g, a, head_dim, head_rows, st);
   }
+  if (!has_tail(p)) return hipSuccess;
   const uint16_t* c = (const uint16_t*)g.C;
   if (p.sub_log2 == 1) {
     hipLaunchKernelGGL((fp8_gemm_4h<true, kEpiPlain, 256, 128, 3>), dim3(p.rem << 1), dim3(256), 0, st,

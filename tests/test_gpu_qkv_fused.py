@@ -295,3 +295,34 @@ def test_less_than_a_round_with_and_without_scratch(with_scratch):
     torch.cuda.synchronize()
     for name, r, o in zip(("q_out", "k_out", "v_out", "ring K", "ring V"), ref, got):
         assert torch.equal(u16_t(r), u16_t(o)), name
+
+
+@pytest.mark.parametrize("M", [1, 3, 1028])  # 192 tiles; five rows of 192 tiles, with 4 rows below whole rounds
+@pytest.mark.parametrize("with_scratch", [True, False])
+def test_many_heads_with_and_without_scratch(M, with_scratch):
+    """128 heads: shapes whose tiles could all take the fused epilogue run without any scratch, also where the scratch
+    would send them, or the rows below whole rounds, through the GEMM and the standalone kernel."""
+    announce("fp8 qkv norm rope many heads", M, with_scratch)
+    import joyomni_ops as jo
+    from joyomni_ops import _lib
+    K, H, D = 512, 128, 128
+    E = H * D
+    a, b, sa, sw, bias, qw, kw, cos, sin = _problem(M, K, H, D, 7 + M, True)
+    need = jo._LIB.joy_fp8_qkv_norm_rope_cache_scratch_size(M, K, H, D)
+    if M < 4 and not with_scratch:
+        assert need >= M * 3 * E * 2
+        return  # fewer than 4 rows do not take the epilogue
+    ref = _outputs(M, H, D, 1, M, 8)
+    got = tuple(t.clone() for t in ref)
+    y = jo.fp8_scaled_mm(a, b, sa, sw, torch.bfloat16, bias)
+    jo.fused_qkv_norm_rope_cache(y, H, 1e-6, qw, kw, cos, sin, ref[0], ref[1], ref[3], ref[4], 0, 0, v_out=ref[2])
+    scratch = torch.empty(max(need, 16) if with_scratch else 16, dtype=torch.uint8, device=DEV)
+    call = lambda: _lib.check(jo._LIB, jo._LIB.joy_fp8_qkv_norm_rope_cache(  # noqa: E731
+        a.data_ptr(), b.data_ptr(), sa.data_ptr(), sw.data_ptr(), bias.data_ptr(), M, K, H, D, 1e-6, qw.data_ptr(),
+        kw.data_ptr(), cos.data_ptr(), sin.data_ptr(), got[0].data_ptr(), E, got[1].data_ptr(), E, got[2].data_ptr(), E,
+        got[3].data_ptr(), got[4].data_ptr(), 1, M, 0, 0, M, 0, scratch.data_ptr() if with_scratch else None,
+        scratch.numel() if with_scratch else 0, torch.cuda.current_stream().cuda_stream))
+    _, names = kernels_of(call)
+    assert not names or (names == [Q4]) == (not with_scratch)
+    for name, r, o in zip(("q_out", "k_out", "v_out", "ring K", "ring V"), ref, got):
+        assert torch.equal(u16_t(r), u16_t(o)), name
