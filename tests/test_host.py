@@ -126,3 +126,15 @@ def test_operator_library_of_another_build_is_an_import_error(source, tmp_path, 
     monkeypatch.setattr(_lib, "TORCH_LIB_PATH", str(path))
     with pytest.raises(ImportError, match="ABI version"):
         _lib.load_ops()
+
+
+def test_operator_library_has_no_thread_local_storage():
+    """A library with a TLS segment loaded into the process slows every access of torch's own thread-local state (1 us an
+    operator), so the operators' library carries none."""
+    import shutil
+    import subprocess
+    from joyomni_ops import _lib
+    if shutil.which("readelf") is None:
+        pytest.skip("readelf not available")
+    out = subprocess.run(["readelf", "-lW", _lib.TORCH_LIB_PATH], capture_output=True, text=True, check=True).stdout
+    assert "LOAD" in out and not any(line.split()[:1] == ["TLS"] for line in out.splitlines())
